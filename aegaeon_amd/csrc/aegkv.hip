@@ -255,12 +255,33 @@ __device__ __forceinline__ void move_chunk16(const char* src, char* dst, uint32_
 }
 
 // A move guard is a word a stream's fence waits set when they give up or
-// see a failed source (aegkv_fence_wait). Guarded kernels read it once at
-// the start, at system scope (it may live in pinned host memory), and move
-// nothing when it is set.
-__device__ __forceinline__ bool guard_set(const uint64_t* guard) {
-  return guard != nullptr &&
-         __hip_atomic_load(guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0;
+// see a failed source (aegkv_fence_wait). The descriptor's staging kernel
+// reads it once per launch, at system scope (it may live in pinned host
+// memory), into a device word behind the descriptor; the moving kernels test
+// that word and move nothing when it is set.
+//
+// Read by every wave of the moving kernel instead, a guard in pinned host
+// memory costs 83-88 ns per wave, one after another whatever the grid: a
+// 12,288-workgroup migration (1.6 GB) took 17.3 ms instead of 0.28, a STAGED
+// gather of 57,600 workgroups 19.1 ms instead of 0.15.
+__device__ __forceinline__ bool guard_set(const uint64_t* __restrict__ seen) {
+  return seen != nullptr && *seen != 0;
+}
+
+// Bring a call's descriptor from the pinned ring to the device (16 B per
+// lane; one launch costs the host the 3 us a small runtime copy does) and
+// take the guard's value along.
+constexpr uint32_t kStageLanes = 256;
+
+__global__ __launch_bounds__(kStageLanes) void desc_stage_kernel(const v4u* __restrict__ host,
+                                                                 v4u* __restrict__ dev,
+                                                                 uint32_t words,
+                                                                 const uint64_t* guard,
+                                                                 uint64_t* seen) {
+  const uint32_t i = blockIdx.x * kStageLanes + threadIdx.x;
+  if (i < words) dev[i] = host[i];
+  if (i == 0 && guard != nullptr)
+    *seen = __hip_atomic_load(guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Byte-granular fallback for callers whose offsets are not 16 B aligned.
@@ -492,6 +513,7 @@ bool valid_copy_unroll(int64_t u) {
 // region whose event was dropped that way (ev == nullptr) has completed.
 struct Ring {
   char* host = nullptr;
+  char* host_dev = nullptr;  // the device's address of `host`
   char* dev = nullptr;
   size_t cap = 0;
   size_t head = 0;
@@ -626,9 +648,13 @@ int ring_grow(Ring& r, size_t need) {
   if (r.dev) AEGKV_HIP(hipFree(r.dev));
   r.host = nullptr;
   r.dev = nullptr;
+  r.cap = 0;
   size_t cap = size_t(4) << 20;
   while (cap < need) cap <<= 1;
   AEGKV_HIP(hipHostMalloc(reinterpret_cast<void**>(&r.host), cap, hipHostMallocDefault));
+  void* mapped = nullptr;
+  AEGKV_HIP(hipHostGetDevicePointer(&mapped, r.host, 0));
+  r.host_dev = static_cast<char*>(mapped);
   AEGKV_HIP(hipMalloc(reinterpret_cast<void**>(&r.dev), cap));
   r.cap = cap;
   r.head = 0;
@@ -684,6 +710,37 @@ int ring_commit(Ring& r, size_t offset, size_t bytes, hipStream_t stream) {
     return hip_fail(e, "hipEventRecord");
   }
   r.inflight.push_back({offset, offset + bytes, sp.ev, stream});
+  return 0;
+}
+
+// A descriptor region in the ring: `bytes` of descriptor (a multiple of 16)
+// and, behind it, the device word that holds the guard's value.
+struct Desc {
+  size_t off = 0;
+  size_t bytes = 0;
+  size_t total() const { return bytes + 16; }
+};
+
+int desc_reserve(Ring& r, size_t bytes, Desc* d) {
+  d->bytes = (bytes + 15) & ~size_t(15);
+  return ring_reserve(r, d->total(), &d->off);
+}
+
+// Enqueue the descriptor's way to the device. *seen: the word the moving
+// kernel tests for `guard`, or null without one.
+int desc_stage(Ring& r, const Desc& d, const uint64_t* guard, const uint64_t** seen,
+               hipStream_t stream) {
+  char* dev = r.dev + d.off;
+  uint64_t* word = guard ? reinterpret_cast<uint64_t*>(dev + d.bytes) : nullptr;
+  const uint32_t words = static_cast<uint32_t>(d.bytes / 16);
+  (void)hipGetLastError();  // clear a stale error: the check below is for this launch
+  hipLaunchKernelGGL(desc_stage_kernel, dim3((words + kStageLanes - 1) / kStageLanes),
+                     dim3(kStageLanes), 0, stream,
+                     reinterpret_cast<const v4u*>(r.host_dev + d.off),
+                     reinterpret_cast<v4u*>(dev), words, guard, word);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return hip_fail(e, "desc_stage_kernel launch");
+  *seen = word;
   return 0;
 }
 
@@ -1121,11 +1178,10 @@ int enqueue_swap_kernel(DeviceCtx* ctx, const SwapLayout& L, const SwapList& E,
   const size_t kpp_off = (seg_bytes + 255) & ~size_t(255);
   const size_t kpp_bytes = sizeof(int64_t) * L.num_groups;
   const size_t ent_off = (kpp_off + kpp_bytes + 255) & ~size_t(255);
-  const size_t total = ent_off + sizeof(EntDesc) * n;
-  size_t off = 0;
-  int rc = ring_reserve(ctx->ring, total, &off);
+  Desc desc;
+  int rc = desc_reserve(ctx->ring, ent_off + sizeof(EntDesc) * n, &desc);
   if (rc) return rc;
-  char* h = ctx->ring.host + off;
+  char* h = ctx->ring.host + desc.off;
   SegDesc* hs = reinterpret_cast<SegDesc*>(h);
   int64_t max_page = 0;
   for (int32_t s = 0; s < S; ++s) {
@@ -1150,32 +1206,34 @@ int enqueue_swap_kernel(DeviceCtx* ctx, const SwapLayout& L, const SwapList& E,
     d.pad = 0;
     he[j] = d;
   }
-  char* dv = ctx->ring.dev + off;
+  char* dv = ctx->ring.dev + desc.off;
   const Tunables t = tunables();
   const ShapeSel sh = swap_shape(t, vec, max_page);
   const int64_t cpt = (max_page + sh.chunk() - 1) / sh.chunk();
   const int64_t items = launch_items(n, S, cpt);
   if (items < 0) {
-    ctx->ring.head = off;  // nothing was enqueued; hand the region back
+    ctx->ring.head = desc.off;  // nothing was enqueued; hand the region back
     return too_many_items(n, S, cpt, "entries");
   }
-  hipError_t e = hipMemcpyAsync(dv, h, total, hipMemcpyHostToDevice, stream);
-  if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(descriptor)");
+  const uint64_t* guard = nullptr;
+  rc = desc_stage(ctx->ring, desc, E.guard, &guard, stream);
+  if (rc) return rc;
   SwapArgs a{reinterpret_cast<const SegDesc*>(dv), reinterpret_cast<const EntDesc*>(dv + ent_off),
              reinterpret_cast<const int64_t*>(dv + kpp_off), static_cast<uint32_t>(S),
              static_cast<uint32_t>(items), static_cast<uint32_t>(cpt), host_side, host_stride,
-             host_rank_off, E.guard};
+             host_rank_off, guard};
   // Non-temporal stores only where the destination is HBM: plain stores to
   // the host pool measured faster (no L2 residency to avoid there).
   const bool nt = t.nt_stores != 0 && !(!is_swap_in && !staged);
-  e = launch_swap(sh, !is_swap_in, vec, nt, launch_grid(wgs, items, sh.wg), stream, a);
+  const hipError_t e =
+      launch_swap(sh, !is_swap_in, vec, nt, launch_grid(wgs, items, sh.wg), stream, a);
   if (e != hipSuccess) {
-    // the descriptor upload is already enqueued: retire its region in order
+    // the descriptor's staging is already enqueued: retire its region in order
     (void)hipGetLastError();
-    (void)ring_commit(ctx->ring, off, total, stream);
+    (void)ring_commit(ctx->ring, desc.off, desc.total(), stream);
     return hip_fail(e, "swap_tiles_kernel launch");
   }
-  return ring_commit(ctx->ring, off, total, stream);
+  return ring_commit(ctx->ring, desc.off, desc.total(), stream);
 }
 
 // A staged chunk with more host runs than this counts as scattered.
@@ -1749,25 +1807,26 @@ int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bas
   rc = get_ctx(&ctx);
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(ctx->mu);
-  const size_t total = copy_pair_offset(num_segments) + sizeof(PairDesc) * num_pairs;
-  size_t off = 0;
-  rc = ring_reserve(ctx->ring, total, &off);
+  Desc desc;
+  rc = desc_reserve(ctx->ring, copy_pair_offset(num_segments) + sizeof(PairDesc) * num_pairs,
+                    &desc);
   if (rc) return rc;
-  char* h = ctx->ring.host + off;
+  char* h = ctx->ring.host + desc.off;
   std::vector<PairDesc> tmp(t.copy_order != 0 ? static_cast<size_t>(num_pairs) : 0);
   pack_copy_desc(h, num_segments, src_bases, dst_bases, page_bytes, num_pairs, src_ids,
                  dst_ids, t.copy_order, tmp.data());
-  char* dv = ctx->ring.dev + off;
-  hipError_t e = hipMemcpyAsync(dv, h, total, hipMemcpyHostToDevice, stream);
-  if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(descriptor)");
-  e = copy_launch(plan, t, ctx->num_cus, num_segments, dv, stream, kind);
+  CopyKind launch = kind;
+  rc = desc_stage(ctx->ring, desc, kind.guard, &launch.guard, stream);
+  if (rc) return rc;
+  const hipError_t e = copy_launch(plan, t, ctx->num_cus, num_segments, ctx->ring.dev + desc.off,
+                                   stream, launch);
   if (e != hipSuccess) {
-    // the descriptor upload is already enqueued: retire its region in order
+    // the descriptor's staging is already enqueued: retire its region in order
     (void)hipGetLastError();
-    (void)ring_commit(ctx->ring, off, total, stream);
+    (void)ring_commit(ctx->ring, desc.off, desc.total(), stream);
     return hip_fail(e, kind.probe ? "copy_probe_kernel launch" : "copy_blocks_kernel launch");
   }
-  return ring_commit(ctx->ring, off, total, stream);
+  return ring_commit(ctx->ring, desc.off, desc.total(), stream);
 }
 
 // ------------------------------------------------ allocation-free copies --
@@ -1959,11 +2018,10 @@ int slices_core(int64_t n, void* const* dst, const void* const* src, const int64
   rc = get_ctx(&ctx);
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(ctx->mu);
-  const size_t total = sizeof(SliceDesc) * keep.size();
-  size_t off = 0;
-  rc = ring_reserve(ctx->ring, total, &off);
+  Desc desc;
+  rc = desc_reserve(ctx->ring, sizeof(SliceDesc) * keep.size(), &desc);
   if (rc) return rc;
-  SliceDesc* h = reinterpret_cast<SliceDesc*>(ctx->ring.host + off);
+  SliceDesc* h = reinterpret_cast<SliceDesc*>(ctx->ring.host + desc.off);
   int64_t first = 0;
   for (size_t k = 0; k < keep.size(); ++k) {
     const int64_t i = keep[k];
@@ -1971,18 +2029,19 @@ int slices_core(int64_t n, void* const* dst, const void* const* src, const int64
                      first};
     first += (bytes[i] + chunk - 1) / chunk;
   }
-  char* dv = ctx->ring.dev + off;
-  hipError_t e = hipMemcpyAsync(dv, h, total, hipMemcpyHostToDevice, stream);
-  if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(descriptor)");
-  e = launch_slices(vec, t.nt_stores != 0, launch_grid(t.swap_in_workgroups, items, 256), stream,
-                    reinterpret_cast<const SliceDesc*>(dv), static_cast<uint32_t>(keep.size()),
-                    static_cast<uint32_t>(items));
+  const uint64_t* guard = nullptr;
+  rc = desc_stage(ctx->ring, desc, nullptr, &guard, stream);
+  if (rc) return rc;
+  const hipError_t e =
+      launch_slices(vec, t.nt_stores != 0, launch_grid(t.swap_in_workgroups, items, 256), stream,
+                    reinterpret_cast<const SliceDesc*>(ctx->ring.dev + desc.off),
+                    static_cast<uint32_t>(keep.size()), static_cast<uint32_t>(items));
   if (e != hipSuccess) {
     (void)hipGetLastError();
-    (void)ring_commit(ctx->ring, off, total, stream);
+    (void)ring_commit(ctx->ring, desc.off, desc.total(), stream);
     return hip_fail(e, "slices_kernel launch");
   }
-  return ring_commit(ctx->ring, off, total, stream);
+  return ring_commit(ctx->ring, desc.off, desc.total(), stream);
 }
 
 }  // namespace

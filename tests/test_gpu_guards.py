@@ -188,6 +188,35 @@ def test_guard_merge_and_guarded_signal(gpu):
         hw.close()
 
 
+@pytest.mark.parametrize("n", [1, 239, 240, 241, 4080, 70000])
+@pytest.mark.parametrize("where", ["host", "device"])
+def test_guarded_migration_with_descriptors_of_any_length(gpu, n, where):
+    """The kernel that brings a descriptor to the device also reads the guard
+    there: with descriptors just below, at and above whole workgroups (one
+    segment: 16 words and one per pair, 256 words a workgroup), short and
+    over a mebibyte, a clear guard moves every pair and a set one none,
+    whether the word lies in pinned host memory or on the device."""
+    _say(f"guarded migration, {n} pairs, guard on the {where}")
+    page = 16
+    g = torch.Generator(device=gpu).manual_seed(n)
+    a = torch.randint(1, 256, (n + 3, page), dtype=torch.uint8, device=gpu, generator=g)
+    b = torch.zeros(n + 5, page, dtype=torch.uint8, device=gpu)
+    rng = np.random.default_rng(n)
+    src, dst = rng.permutation(n + 3)[:n], rng.permutation(n + 5)[:n]
+    words = ops.GuardWords(2) if where == "host" else None
+    guard = words.tensor if words else torch.zeros(2, dtype=torch.int64, device=gpu)
+    guard[1] = 2
+    torch.cuda.synchronize()
+    ops.migrate_blocks([a], [b], src, dst, guard=guard, guard_index=1)
+    torch.cuda.synchronize()
+    assert not b.any(), "a set guard let bytes through"
+    ops.migrate_blocks([a], [b], src, dst, guard=guard, guard_index=0)
+    torch.cuda.synchronize()
+    want = torch.zeros_like(b)
+    want[torch.from_numpy(dst).to(gpu)] = a[torch.from_numpy(src).to(gpu)]
+    assert torch.equal(b, want)
+
+
 @pytest.mark.parametrize("mode", ["direct", "staged"])
 def test_guarded_swaps_in_both_modes(gpu, mode):
     """A set guard stops a swap in either transfer mode: a swap-in moves
