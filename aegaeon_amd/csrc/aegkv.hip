@@ -112,16 +112,14 @@ struct Tunables {
   // swap-out's copies to SDMA and it fell to 29 GB/s (35 one chunk at a
   // time); set bit 0 off for that pattern.
   int64_t staged_overlap = 3;
-  // copy_blocks, 1024-lane shapes with items of >= 32 KiB: LDS reserved per
-  // workgroup so that one workgroup holds a CU (HBM copy rate +1-5 % on
-  // 32-160 KiB tiles; 16 KiB items lose 14 % at one per CU, so they keep 0).
+  // copy_blocks, 1024-lane shapes with items of >= 32 KiB (a fixed unroll):
+  // LDS reserved per workgroup so that one workgroup holds a CU (HBM copy
+  // rate +1-5 % on 32-160 KiB tiles).
   int64_t copy_lds_bytes = int64_t(96) << 10;
   // copy_blocks: the order in which pairs reach the kernel (0: the caller's,
   // 1: by target id, 2: by source id; the checks make the result
-  // order-free). By target id, a copy from one random half of a cache's
-  // blocks to the other runs at 5.98 instead of 5.64 TB/s on 16 KiB tiles,
-  // 5.58 instead of 5.39 on 32 KiB and within 1 % on 64-160 KiB; by source
-  // id it gains about a third as much.
+  // order-free). The kernel's walk (CopyWalk) relies on target order to
+  // write near by; see there for the rates.
   int64_t copy_order = 1;
 };
 Tunables g_tune;
@@ -330,24 +328,54 @@ __global__ __launch_bounds__(WG) void swap_tiles_kernel(
   }
 }
 
-// copy_blocks: item w -> (pair p, segment s, chunk c), pair-major: the
-// workgroups running together move a few pairs across every segment (a
-// segment-major walk, many pairs of one segment at a time, ran 1-9 % slower
-// on 16-160 KiB tiles).
+// The order in which copy_blocks walks its work items, chosen on the host
+// (copy_walk): segment by segment, the pairs of one segment in the order of
+// the descriptor, the chunks of one tile in address order. Workgroups are
+// handed to the 8 XCDs in turn, so items [0, remap_end) are renumbered to
+// give every XCD whole runs of 2^run_shift consecutive items: with pairs in
+// target order each XCD then writes one stretch of one segment at a time.
+//
+// HBM bounds the copy, and this order is what it answers best. Random halves
+// of a cache, against pairs-first items over the whole chip (TB/s, read plus
+// written, 4 KiB items): 160 KiB tiles 5.24 -> 6.45, 64 KiB 5.87 -> 6.19,
+// 32 KiB 5.44 -> 5.88, 20 KiB 5.36 -> 6.01, 16 KiB 5.43 -> 5.99, 4 KiB
+// 5.60 -> 6.15. Segment order alone gives 0-6 % of that, runs alone 2-4 %.
+struct CopyWalk {
+  uint32_t num_pairs;
+  uint32_t num_items;
+  uint32_t chunks_per_tile;
+  uint32_t remap_end;
+  uint32_t run_shift;
+};
+
+struct CopyItem {
+  uint32_t pair, segment, chunk;
+};
+
+__device__ __forceinline__ CopyItem copy_item(const CopyWalk& k, uint32_t w) {
+  if (w < k.remap_end) {
+    const uint32_t r = w & ((8u << k.run_shift) - 1u);
+    w = w - r + ((r & 7u) << k.run_shift) + (r >> 3);
+  }
+  const uint32_t tile = w / k.chunks_per_tile;
+  const uint32_t s = tile / k.num_pairs;
+  return {tile - s * k.num_pairs, s, w - tile * k.chunks_per_tile};
+}
+
+// copy_blocks: one item is one chunk of one (segment, pair) tile. The host
+// keeps num_items + gridDim.x below 2^32 (launch_items).
 template <int WG, int U, bool VEC, bool NT_STORE>
-__global__ __launch_bounds__(WG) void copy_blocks_kernel(
-    const CopySeg* __restrict__ segs, const PairDesc* __restrict__ pairs, uint32_t num_segs,
-    uint32_t num_items, uint32_t chunks_per_tile, const uint64_t* guard) {
+__global__ __launch_bounds__(WG) void copy_blocks_kernel(const CopySeg* __restrict__ segs,
+                                                         const PairDesc* __restrict__ pairs,
+                                                         CopyWalk walk,
+                                                         const uint64_t* __restrict__ guard) {
   constexpr int64_t kChunk = Shape<WG, U>::kChunk;
   if (guard_set(guard)) return;
-  for (uint32_t w = blockIdx.x; w < num_items; w += gridDim.x) {
-    const uint32_t tile = w / chunks_per_tile;
-    const uint32_t c = w - tile * chunks_per_tile;
-    const uint32_t p = tile / num_segs;
-    const uint32_t s = tile - p * num_segs;
-    const PairDesc pr = pairs[p];
-    const CopySeg seg = segs[s];
-    const int64_t begin = static_cast<int64_t>(c) * kChunk;
+  for (uint32_t w = blockIdx.x; w < walk.num_items; w += gridDim.x) {
+    const CopyItem it = copy_item(walk, w);
+    const PairDesc pr = pairs[it.pair];
+    const CopySeg seg = segs[it.segment];
+    const int64_t begin = static_cast<int64_t>(it.chunk) * kChunk;
     if (begin >= seg.page_bytes) continue;
     const uint32_t nbytes = static_cast<uint32_t>(
         (seg.page_bytes - begin < kChunk) ? (seg.page_bytes - begin) : kChunk);
@@ -371,21 +399,19 @@ constexpr int PROBE_READ = 1;
 constexpr int PROBE_WRITE = 2;
 
 template <int WG, int U, int KIND, bool NT_STORE>
-__global__ __launch_bounds__(WG) void copy_probe_kernel(
-    const CopySeg* __restrict__ segs, const PairDesc* __restrict__ pairs, uint32_t num_segs,
-    uint32_t num_items, uint32_t chunks_per_tile, uint32_t* sink, uint32_t magic) {
+__global__ __launch_bounds__(WG) void copy_probe_kernel(const CopySeg* __restrict__ segs,
+                                                        const PairDesc* __restrict__ pairs,
+                                                        CopyWalk walk, uint32_t* sink,
+                                                        uint32_t magic) {
   constexpr int64_t kChunk = Shape<WG, U>::kChunk;
   const uint32_t tid = threadIdx.x;
   v4u acc = {0u, 0u, 0u, 0u};
   const v4u pattern = {tid, blockIdx.x, 0x5a5a5a5au, magic};
-  for (uint32_t w = blockIdx.x; w < num_items; w += gridDim.x) {
-    const uint32_t tile = w / chunks_per_tile;
-    const uint32_t c = w - tile * chunks_per_tile;
-    const uint32_t p = tile / num_segs;
-    const uint32_t s = tile - p * num_segs;
-    const PairDesc pr = pairs[p];
-    const CopySeg seg = segs[s];
-    const int64_t begin = static_cast<int64_t>(c) * kChunk;
+  for (uint32_t w = blockIdx.x; w < walk.num_items; w += gridDim.x) {
+    const CopyItem it = copy_item(walk, w);
+    const PairDesc pr = pairs[it.pair];
+    const CopySeg seg = segs[it.segment];
+    const int64_t begin = static_cast<int64_t>(it.chunk) * kChunk;
     if (begin >= seg.page_bytes) continue;
     const uint32_t n16 = static_cast<uint32_t>(
         ((seg.page_bytes - begin < kChunk) ? (seg.page_bytes - begin) : kChunk) >> 4);
@@ -475,7 +501,8 @@ __global__ __launch_bounds__(kFillBytes / 16) void desc_fill_kernel(FillArgs a) 
   if (i < a.words) a.dst[i] = a.data[i];
 }
 
-// Shapes the library instantiates. 1024-lane shapes move 16 KiB rows; a
+// Shapes that move a whole tile per workgroup (swaps asked for them, copies
+// of more chunks than one launch holds). 1024-lane shapes move 16 KiB rows; a
 // tile that is a multiple of 16 KiB gets the largest U dividing its row
 // count, so one workgroup moves a whole tile (up to 160 KiB) with no tail
 // chunk. Smaller tiles use 256-lane (4 KiB) rows.
@@ -497,6 +524,15 @@ ShapeSel auto_shape(int64_t page) {
   const int64_t small_rows = (page + 4095) / 4096;
   return {256, small_rows <= 1 ? 1 : (small_rows <= 2 ? 2 : 4)};
 }
+
+// Shape of copy_blocks: one load per lane, so an item is 4 KiB, or 1 KiB (one
+// wave) where pages are no multiple of 4 KiB and 4 KiB items would leave
+// lanes idle in the last one. In the order of copy_item, few bytes per item
+// keep what the chip writes at any moment close together: 160 KiB tiles run
+// at 6.45 TB/s with 4 KiB items, 6.18 with 8 or 16 KiB, 6.03 with one item
+// a tile; 12.5 KiB tiles at 5.69 with 4 KiB items and 6.02 with 1 KiB, 1 KiB
+// tiles at 3.84 and 6.19. On multiples of 4 KiB the two are within 1 %.
+ShapeSel copy_shape(int64_t page) { return ShapeSel{page % 4096 == 0 ? 256 : 64, 1}; }
 
 bool valid_copy_unroll(int64_t u) {
   return u == 1 || u == 2 || u == 3 || u == 4 || u == 5 || u == 6 || u == 8 || u == 10;
@@ -859,9 +895,10 @@ bool in_uncached_pool(const void* p) {
 // Workgroups to launch for `items` work items: at most `limit` when limit > 0
 // (the kernels' grid-stride loops cover the rest), else one per item. An HSA
 // dispatch counts work-items in 32 bits, so the grid is also capped at
-// (2^32 - 1) / lanes.
+// (2^32 - 1) / lanes, for narrow workgroups at that of 256 lanes
+// (kMaxLaunchItems), and to whole turns of the 8 XCDs.
 int64_t launch_grid(int64_t limit, int64_t items, int lanes) {
-  const int64_t cap = static_cast<int64_t>(UINT32_MAX) / lanes;
+  const int64_t cap = static_cast<int64_t>(UINT32_MAX) / std::max(lanes, 256) / 8 * 8;
   int64_t g = items;
   if (limit > 0) g = std::min<int64_t>(g, limit);
   return std::max<int64_t>(1, std::min<int64_t>(g, cap));
@@ -869,8 +906,8 @@ int64_t launch_grid(int64_t limit, int64_t items, int lanes) {
 
 // Work items one launch may hold. The kernels walk items with a 32-bit
 // grid-stride loop (w += gridDim.x) and launch_grid caps a grid at
-// (2^32 - 1) / lanes workgroups, so with lanes >= 256 and at most this many
-// items, w + gridDim.x stays below 2^32 and the loop never wraps.
+// (2^32 - 1) / 256 workgroups, so with at most this many items,
+// w + gridDim.x stays below 2^32 and the loop never wraps.
 constexpr int64_t kMaxLaunchItems =
     static_cast<int64_t>(UINT32_MAX) - static_cast<int64_t>(UINT32_MAX) / 256;
 
@@ -939,23 +976,22 @@ hipError_t launch_swap(ShapeSel sh, bool to_host, bool vec, bool nt, int64_t gri
 // caps how many workgroups share a CU.
 template <int WG, int U, bool VEC, bool NT>
 hipError_t launch_copy_t(int64_t grid, unsigned lds, hipStream_t st, const CopySeg* s,
-                         const PairDesc* p, uint32_t ns, uint32_t items, uint32_t cpt,
-                         const uint64_t* guard) {
+                         const PairDesc* p, const CopyWalk& walk, const uint64_t* guard) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
   hipLaunchKernelGGL((copy_blocks_kernel<WG, U, VEC, NT>), dim3(static_cast<uint32_t>(grid)),
-                     dim3(WG), lds, st, s, p, ns, items, cpt, guard);
+                     dim3(WG), lds, st, s, p, walk, guard);
   return hipGetLastError();
 }
 
 hipError_t launch_copy(ShapeSel sh, bool vec, bool nt, int64_t grid, unsigned lds,
-                       hipStream_t st, const CopySeg* s, const PairDesc* p, uint32_t ns,
-                       uint32_t items, uint32_t cpt, const uint64_t* guard) {
-  if (!vec) return launch_copy_t<256, 1, false, false>(grid, 0, st, s, p, ns, items, cpt, guard);
+                       hipStream_t st, const CopySeg* s, const PairDesc* p, const CopyWalk& walk,
+                       const uint64_t* guard) {
+  if (!vec) return launch_copy_t<256, 1, false, false>(grid, 0, st, s, p, walk, guard);
 #define AEGKV_CP(W, UU)                                                               \
   if (sh.wg == W && sh.u == UU)                                                       \
-    return nt ? launch_copy_t<W, UU, true, true>(grid, lds, st, s, p, ns, items, cpt, guard) \
-              : launch_copy_t<W, UU, true, false>(grid, lds, st, s, p, ns, items, cpt, guard);
-  AEGKV_CP(256, 1) AEGKV_CP(256, 2) AEGKV_CP(256, 4) AEGKV_CP(256, 8)
+    return nt ? launch_copy_t<W, UU, true, true>(grid, lds, st, s, p, walk, guard)    \
+              : launch_copy_t<W, UU, true, false>(grid, lds, st, s, p, walk, guard);
+  AEGKV_CP(64, 1) AEGKV_CP(256, 1) AEGKV_CP(256, 2) AEGKV_CP(256, 4) AEGKV_CP(256, 8)
   AEGKV_CP(1024, 1) AEGKV_CP(1024, 2) AEGKV_CP(1024, 3) AEGKV_CP(1024, 4)
   AEGKV_CP(1024, 5) AEGKV_CP(1024, 6) AEGKV_CP(1024, 8) AEGKV_CP(1024, 10)
 #undef AEGKV_CP
@@ -964,28 +1000,27 @@ hipError_t launch_copy(ShapeSel sh, bool vec, bool nt, int64_t grid, unsigned ld
 
 template <int WG, int U, int KIND, bool NT>
 hipError_t launch_probe_t(int64_t grid, unsigned lds, hipStream_t st, const CopySeg* s,
-                          const PairDesc* p, uint32_t ns, uint32_t items, uint32_t cpt,
-                          uint32_t* sink, uint32_t magic) {
+                          const PairDesc* p, const CopyWalk& walk, uint32_t* sink,
+                          uint32_t magic) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
   hipLaunchKernelGGL((copy_probe_kernel<WG, U, KIND, NT>), dim3(static_cast<uint32_t>(grid)),
-                     dim3(WG), lds, st, s, p, ns, items, cpt, sink, magic);
+                     dim3(WG), lds, st, s, p, walk, sink, magic);
   return hipGetLastError();
 }
 
 hipError_t launch_probe(ShapeSel sh, int kind, bool nt, int64_t grid, unsigned lds,
-                        hipStream_t st, const CopySeg* s, const PairDesc* p, uint32_t ns,
-                        uint32_t items, uint32_t cpt, uint32_t* sink, uint32_t magic) {
-#define AEGKV_PR(W, UU)                                                                     \
-  if (sh.wg == W && sh.u == UU) {                                                           \
-    if (kind == PROBE_READ)                                                                 \
-      return launch_probe_t<W, UU, PROBE_READ, false>(grid, lds, st, s, p, ns, items, cpt,  \
-                                                      sink, magic);                         \
-    return nt ? launch_probe_t<W, UU, PROBE_WRITE, true>(grid, lds, st, s, p, ns, items,    \
-                                                         cpt, sink, magic)                  \
-              : launch_probe_t<W, UU, PROBE_WRITE, false>(grid, lds, st, s, p, ns, items,   \
-                                                          cpt, sink, magic);                \
+                        hipStream_t st, const CopySeg* s, const PairDesc* p,
+                        const CopyWalk& walk, uint32_t* sink, uint32_t magic) {
+#define AEGKV_PR(W, UU)                                                                        \
+  if (sh.wg == W && sh.u == UU) {                                                              \
+    if (kind == PROBE_READ)                                                                    \
+      return launch_probe_t<W, UU, PROBE_READ, false>(grid, lds, st, s, p, walk, sink, magic); \
+    return nt ? launch_probe_t<W, UU, PROBE_WRITE, true>(grid, lds, st, s, p, walk, sink,      \
+                                                         magic)                                \
+              : launch_probe_t<W, UU, PROBE_WRITE, false>(grid, lds, st, s, p, walk, sink,     \
+                                                          magic);                              \
   }
-  AEGKV_PR(256, 1) AEGKV_PR(256, 2) AEGKV_PR(256, 4) AEGKV_PR(256, 8)
+  AEGKV_PR(64, 1) AEGKV_PR(256, 1) AEGKV_PR(256, 2) AEGKV_PR(256, 4) AEGKV_PR(256, 8)
   AEGKV_PR(1024, 1) AEGKV_PR(1024, 2) AEGKV_PR(1024, 3) AEGKV_PR(1024, 4)
   AEGKV_PR(1024, 5) AEGKV_PR(1024, 6) AEGKV_PR(1024, 8) AEGKV_PR(1024, 10)
 #undef AEGKV_PR
@@ -1687,20 +1722,36 @@ int copy_check_device(int32_t num_segments, void* const* src_bases, void* const*
 struct CopyPlan {
   ShapeSel sh;
   bool vec;
-  int64_t cpt;    // chunks per tile
-  int64_t items;  // work items (pair x segment x chunk)
+  int64_t items;  // work items (segment x pair x chunk)
+  CopyWalk walk;
 };
+
+// The walk of `items` items (see CopyWalk). Runs hold about 32 tiles: from 8
+// to 512 the rate moves by 2 % (least at 8 and 512 on 4-20 KiB tiles).
+CopyWalk copy_walk(int64_t num_pairs, int64_t cpt, int64_t items) {
+  uint32_t shift = 5;
+  while (shift < 20 && (int64_t(1) << shift) < 32 * cpt) ++shift;
+  const int64_t span = int64_t(8) << shift;
+  return CopyWalk{static_cast<uint32_t>(num_pairs), static_cast<uint32_t>(items),
+                  static_cast<uint32_t>(cpt), static_cast<uint32_t>(items / span * span), shift};
+}
 
 int copy_plan(const Tunables& t, bool vec, int64_t max_page, int32_t num_segments,
               int64_t num_pairs, CopyPlan* out) {
-  ShapeSel sh = auto_shape(max_page);
+  ShapeSel sh = copy_shape(max_page);
   if (t.copy_unroll > 0)
     sh = ShapeSel{t.copy_lanes == 256 ? 256 : 1024, static_cast<int>(t.copy_unroll)};
   if (!vec) sh = ShapeSel{256, 1};
-  const int64_t cpt = (max_page + sh.chunk() - 1) / sh.chunk();
-  const int64_t items = launch_items(num_pairs, num_segments, cpt);
+  int64_t cpt = (max_page + sh.chunk() - 1) / sh.chunk();
+  int64_t items = launch_items(num_pairs, num_segments, cpt);
+  if (items < 0 && vec && t.copy_unroll == 0) {
+    // more small items than one launch holds: whole-tile items
+    sh = auto_shape(max_page);
+    cpt = (max_page + sh.chunk() - 1) / sh.chunk();
+    items = launch_items(num_pairs, num_segments, cpt);
+  }
   if (items < 0) return too_many_items(num_pairs, num_segments, cpt, "pairs");
-  *out = CopyPlan{sh, vec, cpt, items};
+  *out = CopyPlan{sh, vec, items, copy_walk(num_pairs, cpt, items)};
   return 0;
 }
 
@@ -1769,14 +1820,11 @@ hipError_t copy_launch(const CopyPlan& p, const Tunables& t, int num_cus, int32_
                            ? static_cast<unsigned>(t.copy_lds_bytes) : 0u;
   const CopySeg* segs = reinterpret_cast<const CopySeg*>(dv);
   const PairDesc* pairs = reinterpret_cast<const PairDesc*>(dv + copy_pair_offset(num_segments));
-  const uint32_t ns = static_cast<uint32_t>(num_segments);
-  const uint32_t items = static_cast<uint32_t>(p.items);
-  const uint32_t cpt = static_cast<uint32_t>(p.cpt);
   if (kind.probe)
-    return launch_probe(p.sh, kind.probe, t.nt_stores != 0, grid, lds, stream, segs, pairs, ns,
-                        items, cpt, kind.sink, kind.magic);
-  return launch_copy(p.sh, p.vec, t.nt_stores != 0, grid, lds, stream, segs, pairs, ns, items,
-                     cpt, kind.guard);
+    return launch_probe(p.sh, kind.probe, t.nt_stores != 0, grid, lds, stream, segs, pairs,
+                        p.walk, kind.sink, kind.magic);
+  return launch_copy(p.sh, p.vec, t.nt_stores != 0, grid, lds, stream, segs, pairs, p.walk,
+                     kind.guard);
 }
 
 int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bases,

@@ -78,10 +78,11 @@ extern "C" {
 #define AEGKV_TUNE_NT_STORES 5       /* 1: non-temporal stores to HBM     */
 #define AEGKV_TUNE_COPY_WGS_PER_CU 6 /* copy_blocks grid: 0 = one workgroup
                                         per work item, else per-CU count   */
-#define AEGKV_TUNE_COPY_UNROLL 7     /* copy_blocks loads per lane: 0 = from
-                                        the page size, else 1-6, 8 or 10   */
-#define AEGKV_TUNE_SWAP_SHAPE_AUTO 8 /* 1: swap kernels pick their shape
-                                        from the page size like copy_blocks */
+#define AEGKV_TUNE_COPY_UNROLL 7     /* copy_blocks loads per lane: 0 = one, in
+                                        workgroups fit to the page size, else
+                                        1-6, 8 or 10                       */
+#define AEGKV_TUNE_SWAP_SHAPE_AUTO 8 /* 1: swap kernels pick a shape that
+                                        moves a whole page per workgroup   */
 #define AEGKV_TUNE_SWAP_IN_WORKGROUPS 9 /* swap-in kernel: workgroups      */
 #define AEGKV_TUNE_STAGED_DMA_STREAMS 10 /* STAGED copies fan out over this
                                           many library streams (0-4; <= 1:

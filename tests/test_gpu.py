@@ -433,6 +433,39 @@ def test_copy_blocks_every_shape_vs_oracle(gpu, oracle, restore_tuning):
             assert np.array_equal(segs[s].cpu().numpy(), segs_np[s]), (lanes, unroll, wpc, lds, s)
 
 
+@pytest.mark.parametrize("page,segs,pairs", [
+    (4096, 1, 255), (4096, 1, 256), (4096, 1, 257), (4096, 3, 171), (4096, 5, 1),
+    (20480, 1, 409), (20480, 2, 205), (20480, 2, 410), (163840, 2, 33),
+    (16, 7, 300), (1008, 2, 130), (1024, 2, 128), (1040, 2, 200), (3088, 3, 90),
+    (5120, 4, 64), (12800, 3, 79),
+])
+def test_copy_walk_covers_every_item_once(gpu, page, segs, pairs):
+    """The walk renumbers whole turns of 8 runs of items and leaves the rest:
+    item counts just below, at and above such turns, pages of one, several
+    and partly filled items (4 KiB items where the page is a multiple of
+    4 KiB, else 1 KiB), through all three entry points that use it."""
+    _say("copy walk", page, segs, pairs)
+    g = torch.Generator(device=gpu).manual_seed(page + pairs)
+    n = 2 * pairs + 3
+    rng = np.random.default_rng(page + segs + pairs)
+    ids = rng.permutation(n)
+    src, dst = ids[:pairs], ids[pairs:2 * pairs]
+    start = [torch.randint(0, 256, (n, page), dtype=torch.uint8, device=gpu, generator=g)
+             for _ in range(segs)]
+    s, d = torch.from_numpy(src).to(gpu), torch.from_numpy(dst).to(gpu)
+    want = [t.clone().index_copy_(0, d, t[s]) for t in start]
+    for entry in (ops.copy_blocks, ops.copy_blocks_noalloc):
+        got = [t.clone() for t in start]
+        entry(got, src, dst)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), entry.__name__
+    other = [torch.zeros_like(t) for t in start]
+    ops.migrate_blocks(start, other, src, dst)
+    torch.cuda.synchronize()
+    for t, o in zip(start, other):
+        assert torch.equal(o[d], t[s]) and int((o != 0).any(1).sum()) <= pairs
+
+
 @pytest.mark.parametrize("order", [0, 1, 2])
 def test_copy_blocks_pair_orders_vs_oracle(gpu, oracle, restore_tuning, order):
     """The library may hand the kernel the pairs in the caller's order, by
