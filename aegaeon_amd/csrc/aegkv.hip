@@ -213,6 +213,27 @@ struct Shape {
   static constexpr int64_t kChunk = int64_t(WG) * 16 * U;
 };
 
+template <bool NT_STORE>
+__device__ __forceinline__ void store16(gv4u* d, v4u x) {
+  if (NT_STORE)
+    __builtin_nontemporal_store(x, d);
+  else
+    *d = x;
+}
+
+// The guarded U loads of a tail chunk, all issued before the first store.
+// Recursion keeps every value in registers of its own: an array of U values
+// filled under conditions became one wide value that was copied whole at each
+// (252 VGPRs for U = 8, and with 1024 lanes scratch memory: 128 KiB tiles
+// copied at 1.3 TB/s).
+template <int WG, int U, bool NT_STORE>
+__device__ __forceinline__ void move_tail16(const gv4u* s, gv4u* d, uint32_t i, uint32_t n16) {
+  v4u x;
+  if (i < n16) x = __builtin_nontemporal_load(s + i);
+  if constexpr (U > 1) move_tail16<WG, U - 1, NT_STORE>(s, d, i + WG, n16);
+  if (i < n16) store16<NT_STORE>(d + i, x);
+}
+
 // Move nbytes (multiple of 16, at most one chunk) with 16 B per lane. A full
 // chunk issues all U loads back to back before the first store; only a tail
 // chunk pays for per-load guards.
@@ -221,35 +242,15 @@ __device__ __forceinline__ void move_chunk16(const char* src, char* dst, uint32_
   const gv4u* s = (const gv4u*)src;  // generic -> global address space
   gv4u* d = (gv4u*)dst;
   const uint32_t tid = threadIdx.x;
-  v4u r[U];
-  if (nbytes == static_cast<uint32_t>(Shape<WG, U>::kChunk)) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) r[u] = __builtin_nontemporal_load(s + tid + u * WG);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (NT_STORE)
-        __builtin_nontemporal_store(r[u], d + tid + u * WG);
-      else
-        d[tid + u * WG] = r[u];
-    }
+  if (nbytes != static_cast<uint32_t>(Shape<WG, U>::kChunk)) {
+    move_tail16<WG, U, NT_STORE>(s, d, tid, nbytes >> 4);
     return;
   }
-  const uint32_t n16 = nbytes >> 4;
+  v4u r[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const uint32_t i = tid + u * WG;
-    if (i < n16) r[u] = __builtin_nontemporal_load(s + i);
-  }
+  for (int u = 0; u < U; ++u) r[u] = __builtin_nontemporal_load(s + tid + u * WG);
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const uint32_t i = tid + u * WG;
-    if (i < n16) {
-      if (NT_STORE)
-        __builtin_nontemporal_store(r[u], d + i);
-      else
-        d[i] = r[u];
-    }
-  }
+  for (int u = 0; u < U; ++u) store16<NT_STORE>(d + tid + u * WG, r[u]);
 }
 
 // A move guard is a word a stream's fence waits set when they give up or
@@ -532,7 +533,31 @@ ShapeSel auto_shape(int64_t page) {
 // at 6.45 TB/s with 4 KiB items, 6.18 with 8 or 16 KiB, 6.03 with one item
 // a tile; 12.5 KiB tiles at 5.69 with 4 KiB items and 6.02 with 1 KiB, 1 KiB
 // tiles at 3.84 and 6.19. On multiples of 4 KiB the two are within 1 %.
-ShapeSel copy_shape(int64_t page) { return ShapeSel{page % 4096 == 0 ? 256 : 64, 1}; }
+//
+// One load per lane keeps 32 KiB in flight on a CU, which fills the chip's
+// memory system only with all CUs. A stream masked to some of them
+// (aegkv_stream_create_masked) gets more bytes per CU: whole-tile items from
+// 64 KiB, else two loads per lane. On 24 / 16 / 8 of each XCD's 32 CUs, TB/s:
+// 160 KiB tiles 6.07 / 4.52 / 2.40 with one load, 6.09 / 5.34 / 3.09 whole;
+// 64 KiB 5.88 / 4.48 / 2.40, 6.15 / 4.97 / 2.75 whole; 32 KiB 5.47 / 4.33 /
+// 2.38, 5.58 / 5.07 / 2.99 with two.
+ShapeSel copy_shape(int64_t page, bool all_cus) {
+  if (all_cus || page <= 4096) return ShapeSel{page % 4096 == 0 ? 256 : 64, 1};
+  const int64_t row = 1024 * 16;
+  return page >= 4 * row && page % row == 0 ? auto_shape(page) : ShapeSel{256, 2};
+}
+
+// Whether work on `stream` may use every one of the device's CUs (0.3 us).
+bool stream_has_all_cus(hipStream_t stream, int num_cus) {
+  uint32_t mask[32] = {};
+  if (hipExtStreamGetCUMask(stream, 32, mask) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  int n = 0;
+  for (uint32_t m : mask) n += __builtin_popcount(m);
+  return n >= num_cus;
+}
 
 bool valid_copy_unroll(int64_t u) {
   return u == 1 || u == 2 || u == 3 || u == 4 || u == 5 || u == 6 || u == 8 || u == 10;
@@ -1736,9 +1761,9 @@ CopyWalk copy_walk(int64_t num_pairs, int64_t cpt, int64_t items) {
                   static_cast<uint32_t>(cpt), static_cast<uint32_t>(items / span * span), shift};
 }
 
-int copy_plan(const Tunables& t, bool vec, int64_t max_page, int32_t num_segments,
+int copy_plan(const Tunables& t, bool vec, int64_t max_page, bool all_cus, int32_t num_segments,
               int64_t num_pairs, CopyPlan* out) {
-  ShapeSel sh = copy_shape(max_page);
+  ShapeSel sh = copy_shape(max_page, all_cus);
   if (t.copy_unroll > 0)
     sh = ShapeSel{t.copy_lanes == 256 ? 256 : 1024, static_cast<int>(t.copy_unroll)};
   if (!vec) sh = ShapeSel{256, 1};
@@ -1844,7 +1869,7 @@ int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bas
                 "16 B multiples");
   const Tunables t = tunables();
   CopyPlan plan;
-  rc = copy_plan(t, vec, max_page, num_segments, num_pairs, &plan);
+  rc = copy_plan(t, vec, max_page, true, num_segments, num_pairs, &plan);
   if (rc) return rc;
   rc = copy_check_device(num_segments, src_bases, dst_bases, page_bytes, src_num_blocks,
                          dst_num_blocks, same_cache);
@@ -1853,6 +1878,9 @@ int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bas
   if (rc) return rc;
   DeviceCtx* ctx = nullptr;
   rc = get_ctx(&ctx);
+  if (rc) return rc;
+  if (!stream_has_all_cus(stream, ctx->num_cus))
+    rc = copy_plan(t, vec, max_page, false, num_segments, num_pairs, &plan);
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(ctx->mu);
   Desc desc;
@@ -1982,7 +2010,7 @@ int copy_noalloc(int32_t num_segments, void* const* bases, const int64_t* page_b
   if (rc || num_pairs == 0) return rc;
   const Tunables t = tunables();
   CopyPlan plan;
-  rc = copy_plan(t, vec, max_page, num_segments, num_pairs, &plan);
+  rc = copy_plan(t, vec, max_page, true, num_segments, num_pairs, &plan);
   if (rc) return rc;
   rc = copy_check_device(num_segments, bases, bases, page_bytes, num_blocks, num_blocks, true);
   if (rc) return rc;
@@ -1991,6 +2019,9 @@ int copy_noalloc(int32_t num_segments, void* const* bases, const int64_t* page_b
   char* dv = nullptr;
   int num_cus = 0;
   rc = noalloc_scratch(dev, stream, &dv, &num_cus);
+  if (rc) return rc;
+  if (!stream_has_all_cus(stream, num_cus))
+    rc = copy_plan(t, vec, max_page, false, num_segments, num_pairs, &plan);
   if (rc) return rc;
   pack_copy_desc(reinterpret_cast<char*>(g_noalloc_host), num_segments, bases, bases,
                  page_bytes, num_pairs, src_ids, dst_ids, t.copy_order, g_noalloc_order);

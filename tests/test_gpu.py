@@ -376,6 +376,34 @@ def restore_tuning():
         _lib.tune(k, v)
 
 
+@pytest.mark.parametrize("page", [4096, 4112, 8192, 12800, 65536, 65552, 96 << 10, 128 << 10,
+                                  160 << 10, 176 << 10])
+def test_copy_on_a_masked_stream_vs_expectation(gpu, page):
+    """A stream confined to 8 CUs of every XCD takes other copy shapes: two
+    loads per lane or whole tiles, with partly filled last items (12,800 and
+    65,552 bytes) and every loads-per-lane count of the whole-tile shapes."""
+    _say("copy on a masked stream", page)
+    rng = np.random.default_rng(page)
+    n, pairs = 23, 9
+    ids = rng.permutation(n)
+    g = torch.Generator(device=gpu).manual_seed(page)
+    segs = [torch.randint(0, 256, (n, page), dtype=torch.uint8, device=gpu, generator=g)
+            for _ in range(3)]
+    s, d = (torch.from_numpy(x.copy()).to(gpu) for x in (ids[:pairs], ids[pairs:2 * pairs]))
+    want = [t.clone().index_copy_(0, d, t[s]) for t in segs]
+    masked = ops.DedicatedStream(gpu, ops.xcd_cu_mask(8, device=gpu))
+    try:
+        torch.cuda.synchronize()
+        for entry in (ops.copy_blocks, ops.copy_blocks_noalloc):
+            got = [t.clone() for t in segs]
+            torch.cuda.synchronize()
+            entry(got, ids[:pairs], ids[pairs:2 * pairs], stream=masked.stream)
+            masked.stream.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(got, want)), entry.__name__
+    finally:
+        masked.close()
+
+
 @pytest.mark.parametrize("page", [16 * 1024, 64 * 1024, 160 * 1024, 4096, 4000 + 16 * 3])
 def test_copy_probes_touch_only_their_tiles(gpu, page):
     """The read probe changes nothing; the write probe fills exactly the
