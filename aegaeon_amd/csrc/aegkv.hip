@@ -202,6 +202,8 @@ static_assert(sizeof(PairDesc) == 16, "PairDesc layout (descriptors are whole 16
 
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) v4u gv4u;  // global (VM) address space
+typedef v4u v4u_any __attribute__((aligned(1)));     // 16 bytes at any address
+typedef __attribute__((address_space(1))) v4u_any gv4u_any;
 typedef __attribute__((address_space(1))) char gchar;
 
 // A kernel "shape": WG lanes per workgroup, U 16-byte loads in flight per
@@ -283,12 +285,58 @@ __global__ __launch_bounds__(kStageLanes) void desc_stage_kernel(const v4u* __re
     *seen = __hip_atomic_load(guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Byte-granular fallback for callers whose offsets are not 16 B aligned.
-template <int WG>
-__device__ __forceinline__ void move_chunk_bytes(const char* src, char* dst, uint32_t nbytes) {
-  const gchar* s = (const gchar*)src;
-  gchar* d = (gchar*)dst;
-  for (uint32_t i = threadIdx.x; i < nbytes; i += WG) d[i] = s[i];
+// Tiles whose addresses or lengths are no multiples of 16 (a cache whose
+// pages end in a scale, a pool that starts anywhere) are cut into chunks
+// where their *target* crosses 16-byte boundaries: only the first chunk of a
+// tile starts and only its last one ends inside a 16-byte word.
+struct Extent {
+  int64_t begin;
+  uint32_t nbytes;
+};
+
+// Chunk `c` of a `len`-byte tile; the chunk numbered `last` takes the rest.
+template <int64_t kChunk>
+__device__ __forceinline__ Extent any_chunk(const char* dst_tile, int64_t len, uint32_t c,
+                                            uint32_t last) {
+  const int64_t head = static_cast<int64_t>(-reinterpret_cast<uintptr_t>(dst_tile) & 15u);
+  const int64_t begin = c ? head + static_cast<int64_t>(c) * kChunk : 0;
+  const int64_t next = head + (static_cast<int64_t>(c) + 1) * kChunk;
+  const int64_t end = (c == last || next > len) ? len : next;
+  return {begin, begin < end ? static_cast<uint32_t>(end - begin) : 0u};
+}
+
+// Move nbytes from any address to any other: 16 B per lane, loads at the
+// source's own alignment (the hardware takes any) and stores on the target's
+// 16-byte words, with single bytes at both ends. 16,388-byte pages, one byte
+// per lane -> this: block copy 1.7 -> 5.7 TB/s (read plus written), swap-out
+// 34.9 (uncached pool 13.8) -> 51.2 GB/s, swap-in 24.6 -> 52.1, a weight load
+// at odd addresses 24.7 -> 55.4.
+template <int WG, int U, bool NT_STORE>
+__device__ __forceinline__ void move_any(const char* src, char* dst, uint32_t nbytes) {
+  const uint32_t tid = threadIdx.x;
+  uint32_t head = static_cast<uint32_t>(-reinterpret_cast<uintptr_t>(dst)) & 15u;
+  if (head > nbytes) head = nbytes;
+  const uint32_t n16 = (nbytes - head) >> 4;
+  // lanes 0-15 carry the bytes before the first whole word, lanes 16-31
+  // those behind the last one
+  const uint32_t at = tid < 16 ? tid : head + n16 * 16 + (tid - 16);
+  const bool edge = tid < 16 ? tid < head : tid < 32 && at < nbytes;
+  char b = 0;
+  if (edge) b = ((const gchar*)src)[at];
+  const gchar* s = (const gchar*)src + head;
+  gv4u* d = (gv4u*)(dst + head);
+  uint32_t i = tid;
+  for (; i + (U - 1) * WG < n16; i += U * WG) {
+    v4u r[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      r[u] = __builtin_nontemporal_load((const gv4u_any*)(s + (i + u * WG) * 16u));
+#pragma unroll
+    for (int u = 0; u < U; ++u) store16<NT_STORE>(d + i + u * WG, r[u]);
+  }
+  for (; i < n16; i += WG)
+    store16<NT_STORE>(d + i, __builtin_nontemporal_load((const gv4u_any*)(s + i * 16u)));
+  if (edge) ((gchar*)dst)[at] = b;
 }
 
 // Swap tile mover. Item w -> (entry e, segment s, chunk c), entry-major.
@@ -314,18 +362,21 @@ __global__ __launch_bounds__(WG) void swap_tiles_kernel(
     const int64_t unit = seg.page_bytes / kpp[ent.group];
     const int64_t off = unit * ent.first;
     const int64_t len = unit * ent.valid;
-    const int64_t begin = static_cast<int64_t>(c) * kChunk;
-    if (begin >= len) continue;
-    const uint32_t nbytes = static_cast<uint32_t>((len - begin < kChunk) ? (len - begin) : kChunk);
-    char* dev = seg.base + ent.dev_block * seg.page_bytes + off + begin;
+    char* dev = seg.base + ent.dev_block * seg.page_bytes + off;
     char* host = host_base + ent.host_slot * host_stride + host_rank_offset +
-                 seg.host_offset + off + begin;
+                 seg.host_offset + off;
     const char* src = TO_HOST ? dev : host;
     char* dst = TO_HOST ? host : dev;
-    if (VEC)
-      move_chunk16<WG, U, NT_STORE>(src, dst, nbytes);
-    else
-      move_chunk_bytes<WG>(src, dst, nbytes);
+    if (VEC) {
+      const int64_t begin = static_cast<int64_t>(c) * kChunk;
+      if (begin >= len) continue;
+      const uint32_t nbytes =
+          static_cast<uint32_t>((len - begin < kChunk) ? (len - begin) : kChunk);
+      move_chunk16<WG, U, NT_STORE>(src + begin, dst + begin, nbytes);
+    } else {
+      const Extent x = any_chunk<kChunk>(dst, len, c, chunks_per_tile - 1);
+      if (x.nbytes) move_any<WG, U, NT_STORE>(src + x.begin, dst + x.begin, x.nbytes);
+    }
   }
 }
 
@@ -376,16 +427,19 @@ __global__ __launch_bounds__(WG) void copy_blocks_kernel(const CopySeg* __restri
     const CopyItem it = copy_item(walk, w);
     const PairDesc pr = pairs[it.pair];
     const CopySeg seg = segs[it.segment];
-    const int64_t begin = static_cast<int64_t>(it.chunk) * kChunk;
-    if (begin >= seg.page_bytes) continue;
-    const uint32_t nbytes = static_cast<uint32_t>(
-        (seg.page_bytes - begin < kChunk) ? (seg.page_bytes - begin) : kChunk);
-    const char* src = seg.src + pr.src * seg.page_bytes + begin;
-    char* dst = seg.dst + pr.dst * seg.page_bytes + begin;
-    if (VEC)
-      move_chunk16<WG, U, NT_STORE>(src, dst, nbytes);
-    else
-      move_chunk_bytes<WG>(src, dst, nbytes);
+    const char* src = seg.src + pr.src * seg.page_bytes;
+    char* dst = seg.dst + pr.dst * seg.page_bytes;
+    if (VEC) {
+      const int64_t begin = static_cast<int64_t>(it.chunk) * kChunk;
+      if (begin >= seg.page_bytes) continue;
+      const uint32_t nbytes = static_cast<uint32_t>(
+          (seg.page_bytes - begin < kChunk) ? (seg.page_bytes - begin) : kChunk);
+      move_chunk16<WG, U, NT_STORE>(src + begin, dst + begin, nbytes);
+    } else {
+      const Extent x =
+          any_chunk<kChunk>(dst, seg.page_bytes, it.chunk, walk.chunks_per_tile - 1);
+      if (x.nbytes) move_any<WG, U, NT_STORE>(src + x.begin, dst + x.begin, x.nbytes);
+    }
   }
 }
 
@@ -474,13 +528,17 @@ __global__ __launch_bounds__(WG) void slices_kernel(const SliceDesc* __restrict_
         hi = mid - 1;
     }
     const SliceDesc sl = slices[lo];
-    const int64_t begin = (static_cast<int64_t>(w) - sl.first_item) * kChunk;
-    const uint32_t nbytes =
-        static_cast<uint32_t>((sl.bytes - begin < kChunk) ? (sl.bytes - begin) : kChunk);
-    if (VEC)
+    const uint32_t c = static_cast<uint32_t>(static_cast<int64_t>(w) - sl.first_item);
+    if (VEC) {
+      const int64_t begin = static_cast<int64_t>(c) * kChunk;
+      const uint32_t nbytes =
+          static_cast<uint32_t>((sl.bytes - begin < kChunk) ? (sl.bytes - begin) : kChunk);
       move_chunk16<WG, U, NT_STORE>(sl.src + begin, sl.dst + begin, nbytes);
-    else
-      move_chunk_bytes<WG>(sl.src + begin, sl.dst + begin, nbytes);
+    } else {
+      const uint32_t last = static_cast<uint32_t>((sl.bytes - 1) / kChunk);
+      const Extent x = any_chunk<kChunk>(sl.dst, sl.bytes, c, last);
+      if (x.nbytes) move_any<WG, U, NT_STORE>(sl.src + x.begin, sl.dst + x.begin, x.nbytes);
+    }
   }
 }
 
@@ -985,9 +1043,13 @@ hipError_t launch_swap_shape(bool to_host, bool nt, int64_t grid, hipStream_t st
 
 hipError_t launch_swap(ShapeSel sh, bool to_host, bool vec, bool nt, int64_t grid,
                        hipStream_t st, const SwapArgs& a) {
-  if (!vec)
-    return to_host ? launch_swap_t<256, 1, true, false, false>(grid, st, a)
-                   : launch_swap_t<256, 1, false, false, false>(grid, st, a);
+  if (!vec) {
+    if (to_host)
+      return nt ? launch_swap_t<256, 2, true, false, true>(grid, st, a)
+                : launch_swap_t<256, 2, true, false, false>(grid, st, a);
+    return nt ? launch_swap_t<256, 2, false, false, true>(grid, st, a)
+              : launch_swap_t<256, 2, false, false, false>(grid, st, a);
+  }
 #define AEGKV_SW(W, UU) \
   if (sh.wg == W && sh.u == UU) return launch_swap_shape<W, UU>(to_host, nt, grid, st, a);
   AEGKV_SW(256, 1) AEGKV_SW(256, 2) AEGKV_SW(256, 4)
@@ -1011,7 +1073,13 @@ hipError_t launch_copy_t(int64_t grid, unsigned lds, hipStream_t st, const CopyS
 hipError_t launch_copy(ShapeSel sh, bool vec, bool nt, int64_t grid, unsigned lds,
                        hipStream_t st, const CopySeg* s, const PairDesc* p, const CopyWalk& walk,
                        const uint64_t* guard) {
-  if (!vec) return launch_copy_t<256, 1, false, false>(grid, 0, st, s, p, walk, guard);
+  if (!vec) {
+    if (sh.wg == 64)
+      return nt ? launch_copy_t<64, 1, false, true>(grid, 0, st, s, p, walk, guard)
+                : launch_copy_t<64, 1, false, false>(grid, 0, st, s, p, walk, guard);
+    return nt ? launch_copy_t<256, 1, false, true>(grid, 0, st, s, p, walk, guard)
+              : launch_copy_t<256, 1, false, false>(grid, 0, st, s, p, walk, guard);
+  }
 #define AEGKV_CP(W, UU)                                                               \
   if (sh.wg == W && sh.u == UU)                                                       \
     return nt ? launch_copy_t<W, UU, true, true>(grid, lds, st, s, p, walk, guard)    \
@@ -1056,8 +1124,11 @@ hipError_t launch_slices(bool vec, bool nt, int64_t grid, hipStream_t st,
                          const SliceDesc* slices, uint32_t num_slices, uint32_t items) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
   const dim3 g(static_cast<uint32_t>(grid));
-  if (!vec)
-    hipLaunchKernelGGL((slices_kernel<256, 1, false, false>), g, dim3(256), 0, st, slices,
+  if (!vec && nt)
+    hipLaunchKernelGGL((slices_kernel<256, 2, false, true>), g, dim3(256), 0, st, slices,
+                       num_slices, items);
+  else if (!vec)
+    hipLaunchKernelGGL((slices_kernel<256, 2, false, false>), g, dim3(256), 0, st, slices,
                        num_slices, items);
   else if (nt)
     hipLaunchKernelGGL((slices_kernel<256, 2, true, true>), g, dim3(256), 0, st, slices,
@@ -1211,10 +1282,10 @@ int validate_list(const SwapLayout& L, const SwapList& E, bool is_swap_in) {
 }
 
 // Launch shape of the swap kernels: 256 lanes with the tuned loads per
-// lane, or (tuning key 8) the copy's page-sized shape; bytes alone on the
-// unaligned path.
+// lane, or (tuning key 8) a whole-tile shape; two loads where addresses or
+// lengths are no multiples of 16.
 ShapeSel swap_shape(const Tunables& t, bool vec, int64_t max_page) {
-  if (!vec) return ShapeSel{256, 1};
+  if (!vec) return ShapeSel{256, 2};
   return t.swap_shape_auto ? auto_shape(max_page)
                            : ShapeSel{256, static_cast<int>(t.swap_unroll)};
 }
@@ -1766,13 +1837,17 @@ int copy_plan(const Tunables& t, bool vec, int64_t max_page, bool all_cus, int32
   ShapeSel sh = copy_shape(max_page, all_cus);
   if (t.copy_unroll > 0)
     sh = ShapeSel{t.copy_lanes == 256 ? 256 : 1024, static_cast<int>(t.copy_unroll)};
-  if (!vec) sh = ShapeSel{256, 1};
-  int64_t cpt = (max_page + sh.chunk() - 1) / sh.chunk();
+  auto chunks = [&] { return (max_page + sh.chunk() - 1) / sh.chunk(); };
+  // unaligned tiles: the last chunk takes up to half a chunk more, so that
+  // a few bytes over do not cost a wave of their own
+  auto any_chunks = [&] { return std::max<int64_t>(1, (max_page + sh.chunk() / 2) / sh.chunk()); };
+  if (!vec) sh = ShapeSel{64, 1};
+  int64_t cpt = vec ? chunks() : any_chunks();
   int64_t items = launch_items(num_pairs, num_segments, cpt);
-  if (items < 0 && vec && t.copy_unroll == 0) {
-    // more small items than one launch holds: whole-tile items
-    sh = auto_shape(max_page);
-    cpt = (max_page + sh.chunk() - 1) / sh.chunk();
+  if (items < 0 && (!vec || t.copy_unroll == 0)) {
+    // more small items than one launch holds
+    sh = vec ? auto_shape(max_page) : ShapeSel{256, 1};
+    cpt = vec ? chunks() : any_chunks();
     items = launch_items(num_pairs, num_segments, cpt);
   }
   if (items < 0) return too_many_items(num_pairs, num_segments, cpt, "pairs");
@@ -2071,7 +2146,7 @@ int slices_core(int64_t n, void* const* dst, const void* const* src, const int64
                   static_cast<long long>(a), static_cast<long long>(b));
   }
   if (keep.empty()) return 0;
-  const int64_t chunk = vec ? int64_t(256) * 16 * 2 : int64_t(256) * 16;
+  const int64_t chunk = int64_t(256) * 16 * 2;
   int64_t items = 0;
   for (int64_t i : keep) {
     items += (bytes[i] + chunk - 1) / chunk;

@@ -404,6 +404,82 @@ def test_copy_on_a_masked_stream_vs_expectation(gpu, page):
         masked.close()
 
 
+def _shifted(nbytes, shift, device, g):
+    """Random device bytes starting `shift` bytes behind a 16-byte boundary,
+    with 64 bytes around them that no move may touch: (all, the view)."""
+    whole = torch.randint(0, 256, (64 + shift + nbytes + 64,), dtype=torch.uint8, device=device,
+                          generator=g)
+    return whole, whole[64 + shift:64 + shift + nbytes]
+
+
+@pytest.mark.parametrize("shift", [0, 1, 7, 8, 15])
+@pytest.mark.parametrize("page", [1, 15, 17, 33, 1023, 1535, 1536, 1537, 2047, 4099, 8191, 8209,
+                                  16388, 24583])
+def test_moves_at_any_alignment(gpu, page, shift):
+    """Pages and starts that are no multiples of 16 bytes: every entry point
+    that moves bytes, with targets at many offsets into their 16-byte words
+    (odd pages give each block another), pages around the sizes where the
+    last chunk takes the rest of the tile, and nothing outside the target
+    pages touched."""
+    _say("any alignment", page, shift)
+    g = torch.Generator(device=gpu).manual_seed(page * 16 + shift)
+    rng = np.random.default_rng(page + shift)
+    n, m = 40, 17
+    ids = rng.permutation(n)
+    src, dst = ids[:m], ids[m:2 * m]
+    s, d = torch.from_numpy(src.copy()).to(gpu), torch.from_numpy(dst.copy()).to(gpu)
+    whole, flat = _shifted(n * page, shift, gpu, g)
+    start = whole.clone()
+    seg = flat.view(n, page)
+
+    def expect(rows):
+        want = start.clone()
+        want[64 + shift:64 + shift + n * page].view(n, page)[d] = rows
+        return want
+
+    rows = seg[s].clone()
+    for entry in (ops.copy_blocks, ops.copy_blocks_noalloc):
+        whole.copy_(start)
+        entry([seg], src, dst)
+        torch.cuda.synchronize()
+        assert torch.equal(whole, expect(rows)), entry.__name__
+    whole.copy_(start)
+    _, peer = _shifted(n * page, (shift + 5) % 16, gpu, g)
+    peer = peer.view(n, page)
+    ops.migrate_blocks([peer], [seg], src, dst)
+    torch.cuda.synchronize()
+    assert torch.equal(whole, expect(peer[s])), "migrate"
+    # swap-in of rows the host holds, then out again to other host blocks
+    pool = ops.PinnedHostPool(128 + 16 + n * page)
+    pool.tensor.random_()
+    host = pool.tensor[64 + 3:64 + 3 + n * page]
+    before = pool.tensor.clone()
+    kept = host.view(n, page)[torch.from_numpy(src.copy())].to(gpu)
+    for mode in ("direct", "staged"):
+        whole.copy_(start)
+        pool.tensor.copy_(before)
+        torch.cuda.synchronize()
+        ops.swap(src, dst, True, seg, host, mode=mode)
+        torch.cuda.synchronize()
+        assert torch.equal(whole, expect(kept)), f"swap-in {mode}"
+        ops.swap(dst, dst, False, seg, host, mode=mode)
+        torch.cuda.synchronize()
+        want = before.clone()
+        want[67:67 + n * page].view(n, page)[torch.from_numpy(dst.copy())] = kept.cpu()
+        assert torch.equal(pool.tensor, want), f"swap-out {mode}"
+    # weight slices of several lengths at odd places
+    whole.copy_(start)
+    cuts = [0, 1, page, page + 9, 3 * page, n * page]
+    cuts = sorted({c for c in cuts if c <= n * page})
+    torch.cuda.synchronize()
+    ops.load_slices([flat[a:b] for a, b in zip(cuts, cuts[1:])],
+                    [host[a:b] for a, b in zip(cuts, cuts[1:])])
+    torch.cuda.synchronize()
+    want = start.clone()
+    want[64 + shift:64 + shift + n * page] = host.to(gpu)
+    assert torch.equal(whole, want), "slices"
+
+
 @pytest.mark.parametrize("page", [16 * 1024, 64 * 1024, 160 * 1024, 4096, 4000 + 16 * 3])
 def test_copy_probes_touch_only_their_tiles(gpu, page):
     """The read probe changes nothing; the write probe fills exactly the
