@@ -31,6 +31,7 @@
 
 #include <algorithm>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -416,31 +417,71 @@ __device__ __forceinline__ CopyItem copy_item(const CopyWalk& k, uint32_t w) {
 
 // copy_blocks: one item is one chunk of one (segment, pair) tile. The host
 // keeps num_items + gridDim.x below 2^32 (launch_items).
+template <int WG, int U, bool VEC, bool NT_STORE, typename Segs, typename Pairs>
+__device__ __forceinline__ void copy_items(Segs segs, Pairs pairs, const CopyWalk& walk) {
+  constexpr int64_t kChunk = Shape<WG, U>::kChunk;
+  for (uint32_t w = blockIdx.x; w < walk.num_items; w += gridDim.x) {
+    const CopyItem it = copy_item(walk, w);
+    const int64_t src_block = pairs[it.pair].src, dst_block = pairs[it.pair].dst;
+    const int64_t page = segs[it.segment].page_bytes;
+    const char* src = segs[it.segment].src + src_block * page;
+    char* dst = segs[it.segment].dst + dst_block * page;
+    // both descriptor entries are wanted at once, not the addresses only
+    // behind a branch on the page's size (two trips through the scalar cache)
+    asm("" : "+s"(src), "+s"(dst));
+    if (VEC) {
+      const int64_t begin = static_cast<int64_t>(it.chunk) * kChunk;
+      if (begin >= page) continue;
+      const uint32_t nbytes =
+          static_cast<uint32_t>((page - begin < kChunk) ? (page - begin) : kChunk);
+      move_chunk16<WG, U, NT_STORE>(src + begin, dst + begin, nbytes);
+    } else {
+      const Extent x = any_chunk<kChunk>(dst, page, it.chunk, walk.chunks_per_tile - 1);
+      if (x.nbytes) move_any<WG, U, NT_STORE>(src + x.begin, dst + x.begin, x.nbytes);
+    }
+  }
+}
+
 template <int WG, int U, bool VEC, bool NT_STORE>
 __global__ __launch_bounds__(WG) void copy_blocks_kernel(const CopySeg* __restrict__ segs,
                                                          const PairDesc* __restrict__ pairs,
                                                          CopyWalk walk,
                                                          const uint64_t* __restrict__ guard) {
-  constexpr int64_t kChunk = Shape<WG, U>::kChunk;
   if (guard_set(guard)) return;
-  for (uint32_t w = blockIdx.x; w < walk.num_items; w += gridDim.x) {
-    const CopyItem it = copy_item(walk, w);
-    const PairDesc pr = pairs[it.pair];
-    const CopySeg seg = segs[it.segment];
-    const char* src = seg.src + pr.src * seg.page_bytes;
-    char* dst = seg.dst + pr.dst * seg.page_bytes;
-    if (VEC) {
-      const int64_t begin = static_cast<int64_t>(it.chunk) * kChunk;
-      if (begin >= seg.page_bytes) continue;
-      const uint32_t nbytes = static_cast<uint32_t>(
-          (seg.page_bytes - begin < kChunk) ? (seg.page_bytes - begin) : kChunk);
-      move_chunk16<WG, U, NT_STORE>(src + begin, dst + begin, nbytes);
-    } else {
-      const Extent x =
-          any_chunk<kChunk>(dst, seg.page_bytes, it.chunk, walk.chunks_per_tile - 1);
-      if (x.nbytes) move_any<WG, U, NT_STORE>(src + x.begin, dst + x.begin, x.nbytes);
-    }
-  }
+  copy_items<WG, U, VEC, NT_STORE>(segs, pairs, walk);
+}
+
+// A short copy's whole descriptor (segment table, then pair table) in the
+// kernel's own arguments, which the runtime copies when the launch is
+// enqueued (a graph that captures it keeps its own copy) and every workgroup
+// reads through the scalar cache: the call is one launch, with no upload in
+// front of it, no ring region and no event behind it.
+// Copying one block of 72 segments takes the host 8 us through the library
+// instead of 14 and the caller 19 instead of 22 until it is done; 63 blocks of
+// 72 x 32 KiB take 54 us a pass instead of 61.
+// kInlineBytes keeps all arguments, hidden ones among them, within 4 KiB: 72
+// segments and 94 pairs.
+constexpr uint32_t kInlineBytes = 3808;
+struct alignas(16) InlineCopy {
+  CopyWalk walk;
+  uint32_t pair_offset;  // bytes of the segment table
+  uint32_t pad[2];
+  unsigned char data[kInlineBytes];
+};
+static_assert(offsetof(InlineCopy, data) == 32 && sizeof(InlineCopy) <= 4096,
+              "InlineCopy layout");
+typedef __attribute__((address_space(4))) const char kernarg_char;
+typedef __attribute__((address_space(4))) const CopySeg kernarg_seg;
+typedef __attribute__((address_space(4))) const PairDesc kernarg_pair;
+
+template <int WG, bool VEC, bool NT_STORE>
+__global__ __launch_bounds__(WG) void copy_blocks_inline_kernel(InlineCopy a) {
+  // the tables are indexed where the launch put them: `a` is the kernel's
+  // only argument and starts its argument segment
+  kernarg_char* data =
+      (kernarg_char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(InlineCopy, data);
+  copy_items<WG, 1, VEC, NT_STORE>((kernarg_seg*)data, (kernarg_pair*)(data + a.pair_offset),
+                                   a.walk);
 }
 
 // Measurement twins of copy_blocks_kernel (aegkv_copy_probe): the same
@@ -542,22 +583,54 @@ __global__ __launch_bounds__(WG) void slices_kernel(const SliceDesc* __restrict_
   }
 }
 
-// Descriptor bytes carried in one launch's kernel arguments (allocation-free
-// copies): lane i stores the i-th 16 bytes. The runtime copies a launch's
-// arguments when the launch is enqueued, and a graph that captures the
-// launch keeps its own copy, so the host buffer they came from is free as
-// soon as the launch call returns.
-constexpr uint32_t kFillBytes = 2048;
-struct FillArgs {
-  v4u data[kFillBytes / 16];
-  v4u* dst;
-  uint32_t words;  // 16-byte words to store, <= kFillBytes / 16
-  uint32_t pad;
+// A part of an allocation-free copy's descriptor in one launch's kernel
+// arguments, packed, and unpacked into the tables by the launch: 16 bytes a
+// segment (address and page), then 8 bytes a pair (32-bit ids; 16 bytes where
+// a cache has more blocks than those name). The runtime copies a launch's
+// arguments when the launch is enqueued, and a graph that captures the launch
+// keeps its own copy, so the host buffer they came from is free as soon as the
+// launch call returns.
+//
+// One such launch takes 4.9 us on the stream whatever it carries, so they
+// carry all that 4 KiB of arguments hold (hidden ones among them): 72
+// segments and 600 pairs go out in two launches, where 2 KiB of finished
+// table entries a launch took six.
+constexpr uint32_t kFillBytes = 3776;
+constexpr uint32_t kFillLanes = 512;
+struct FillSeg {
+  char* base;
+  int64_t page_bytes;
 };
+struct FillPair {
+  uint32_t src, dst;
+};
+struct alignas(16) FillArgs {
+  CopySeg* segs;
+  PairDesc* pairs;
+  uint32_t num_segs;
+  uint32_t num_pairs;
+  uint32_t wide;  // pairs are PairDesc
+  uint32_t pad;
+  unsigned char data[kFillBytes];
+};
+static_assert(kFillBytes / sizeof(FillPair) <= kFillLanes &&
+              offsetof(FillArgs, data) % 16 == 0 && kFillBytes % 16 == 0, "FillArgs layout");
 
-__global__ __launch_bounds__(kFillBytes / 16) void desc_fill_kernel(FillArgs a) {
+__global__ __launch_bounds__(kFillLanes) void desc_fill_kernel(FillArgs a) {
   const uint32_t i = threadIdx.x;
-  if (i < a.words) a.dst[i] = a.data[i];
+  if (i < a.num_segs) {
+    const FillSeg s = reinterpret_cast<const FillSeg*>(a.data)[i];
+    a.segs[i] = CopySeg{s.base, s.base, s.page_bytes, 0};
+  }
+  const unsigned char* pairs = a.data + a.num_segs * sizeof(FillSeg);
+  if (i < a.num_pairs) {
+    if (a.wide) {
+      a.pairs[i] = reinterpret_cast<const PairDesc*>(pairs)[i];
+    } else {
+      const FillPair p = reinterpret_cast<const FillPair*>(pairs)[i];
+      a.pairs[i] = PairDesc{p.src, p.dst};
+    }
+  }
 }
 
 // Shapes that move a whole tile per workgroup (swaps asked for them, copies
@@ -1089,6 +1162,26 @@ hipError_t launch_copy(ShapeSel sh, bool vec, bool nt, int64_t grid, unsigned ld
   AEGKV_CP(1024, 5) AEGKV_CP(1024, 6) AEGKV_CP(1024, 8) AEGKV_CP(1024, 10)
 #undef AEGKV_CP
   return hipErrorInvalidValue;
+}
+
+template <int WG, bool VEC, bool NT>
+hipError_t launch_inline_t(int64_t grid, hipStream_t st, const InlineCopy& a) {
+  (void)hipGetLastError();  // clear a stale error: the check below is for this launch
+  hipLaunchKernelGGL((copy_blocks_inline_kernel<WG, VEC, NT>),
+                     dim3(static_cast<uint32_t>(grid)), dim3(WG), 0, st, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_inline(int lanes, bool vec, bool nt, int64_t grid, hipStream_t st,
+                         const InlineCopy& a) {
+  if (!vec)
+    return nt ? launch_inline_t<64, false, true>(grid, st, a)
+              : launch_inline_t<64, false, false>(grid, st, a);
+  if (lanes == 64)
+    return nt ? launch_inline_t<64, true, true>(grid, st, a)
+              : launch_inline_t<64, true, false>(grid, st, a);
+  return nt ? launch_inline_t<256, true, true>(grid, st, a)
+            : launch_inline_t<256, true, false>(grid, st, a);
 }
 
 template <int WG, int U, int KIND, bool NT>
@@ -1885,7 +1978,7 @@ void sort_pairs(PairDesc* a, int64_t n, bool by_dst, PairDesc* tmp) {
   if (from != a) std::copy(from, from + n, a);
 }
 
-void pack_copy_desc(char* h, int32_t num_segments, void* const* src_bases,
+void pack_copy_desc(char* h, size_t pair_offset, int32_t num_segments, void* const* src_bases,
                     void* const* dst_bases, const int64_t* page_bytes, int64_t num_pairs,
                     const int64_t* src_ids, const int64_t* dst_ids, int64_t order,
                     PairDesc* tmp) {
@@ -1893,7 +1986,7 @@ void pack_copy_desc(char* h, int32_t num_segments, void* const* src_bases,
   for (int32_t s = 0; s < num_segments; ++s)
     hs[s] = CopySeg{static_cast<const char*>(src_bases[s]), static_cast<char*>(dst_bases[s]),
                     page_bytes[s], 0};
-  PairDesc* hp = reinterpret_cast<PairDesc*>(h + copy_pair_offset(num_segments));
+  PairDesc* hp = reinterpret_cast<PairDesc*>(h + pair_offset);
   for (int64_t i = 0; i < num_pairs; ++i) hp[i] = PairDesc{src_ids[i], dst_ids[i]};
   // Targets are distinct and never sources, so any order gives the same
   // result. Copies of small tiles run faster with their targets in order:
@@ -1927,6 +2020,33 @@ hipError_t copy_launch(const CopyPlan& p, const Tunables& t, int num_cus, int32_
                      kind.guard);
 }
 
+// A copy whose descriptor fits a launch's arguments goes out as that one
+// launch, in the shapes of the whole chip (one load per lane). *launched:
+// whether it did.
+int copy_inline(const CopyPlan& p, const Tunables& t, int num_cus, int32_t num_segments,
+                void* const* src_bases, void* const* dst_bases, const int64_t* page_bytes,
+                int64_t num_pairs, const int64_t* src_ids, const int64_t* dst_ids,
+                hipStream_t stream, bool* launched) {
+  const size_t pair_offset = sizeof(CopySeg) * static_cast<size_t>(num_segments);
+  *launched = false;
+  if (p.sh.u != 1 || p.sh.wg > 256 || (!p.vec && p.sh.wg != 64) ||
+      pair_offset >= kInlineBytes ||
+      num_pairs > static_cast<int64_t>((kInlineBytes - pair_offset) / sizeof(PairDesc)))
+    return 0;
+  InlineCopy a;
+  a.walk = p.walk;
+  a.pair_offset = static_cast<uint32_t>(pair_offset);
+  a.pad[0] = a.pad[1] = 0;
+  PairDesc tmp[kInlineBytes / sizeof(PairDesc)];
+  pack_copy_desc(reinterpret_cast<char*>(a.data), pair_offset, num_segments, src_bases, dst_bases,
+                 page_bytes, num_pairs, src_ids, dst_ids, t.copy_order, tmp);
+  const int64_t grid = launch_grid(t.copy_wgs_per_cu * num_cus, p.items, p.sh.wg);
+  const hipError_t e = launch_inline(p.sh.wg, p.vec, t.nt_stores != 0, grid, stream, a);
+  if (e != hipSuccess) return hip_fail(e, "copy_blocks_inline_kernel launch");
+  *launched = true;
+  return 0;
+}
+
 int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bases,
               const int64_t* page_bytes, int64_t src_num_blocks, int64_t dst_num_blocks,
               int64_t num_pairs, const int64_t* src_ids, const int64_t* dst_ids, bool same_cache,
@@ -1957,6 +2077,12 @@ int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bas
   if (!stream_has_all_cus(stream, ctx->num_cus))
     rc = copy_plan(t, vec, max_page, false, num_segments, num_pairs, &plan);
   if (rc) return rc;
+  if (!kind.probe && !kind.guard) {
+    bool launched = false;
+    rc = copy_inline(plan, t, ctx->num_cus, num_segments, src_bases, dst_bases, page_bytes,
+                     num_pairs, src_ids, dst_ids, stream, &launched);
+    if (rc || launched) return rc;
+  }
   std::lock_guard<std::mutex> lk(ctx->mu);
   Desc desc;
   rc = desc_reserve(ctx->ring, copy_pair_offset(num_segments) + sizeof(PairDesc) * num_pairs,
@@ -1964,8 +2090,8 @@ int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bas
   if (rc) return rc;
   char* h = ctx->ring.host + desc.off;
   std::vector<PairDesc> tmp(t.copy_order != 0 ? static_cast<size_t>(num_pairs) : 0);
-  pack_copy_desc(h, num_segments, src_bases, dst_bases, page_bytes, num_pairs, src_ids,
-                 dst_ids, t.copy_order, tmp.data());
+  pack_copy_desc(h, copy_pair_offset(num_segments), num_segments, src_bases, dst_bases,
+                 page_bytes, num_pairs, src_ids, dst_ids, t.copy_order, tmp.data());
   CopyKind launch = kind;
   rc = desc_stage(ctx->ring, desc, kind.guard, &launch.guard, stream);
   if (rc) return rc;
@@ -1986,8 +2112,8 @@ int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bas
 // allocate. The descriptor (segment table + pair table) goes to `scratch`,
 // a fixed device array every GPU holds for the life of the process, instead
 // of the library's upload ring; it travels in the kernel arguments of small
-// fill launches (2 KiB each), so a graph that captures the call replays its
-// own descriptor. The ids are checked with fixed host arrays instead of a
+// fill launches, or of the copy itself where it is short (copy_inline), so a
+// graph that captures the call replays its own descriptor. The ids are checked with fixed host arrays instead of a
 // block-indexed map. Nothing is allocated on the host or the device. Every
 // call on a device shares that device's array, so calls that overlap on one
 // device (different streams, or threads, or a graph replayed beside other
@@ -2045,18 +2171,40 @@ int noalloc_scratch(int dev, hipStream_t stream, char** out, int* num_cus) {
   return 0;
 }
 
-// dst[0, bytes) <- src[0, bytes) on `stream`, kFillBytes per launch of
-// desc_fill_kernel (bytes is a multiple of 16; descriptors are).
-hipError_t noalloc_fill(char* dst, const unsigned char* src, size_t bytes, hipStream_t stream) {
+// The tables packed at g_noalloc_host to their places in `scratch`, kFillBytes
+// of packed entries a launch of desc_fill_kernel.
+hipError_t noalloc_fill(char* dst, const unsigned char* src, int32_t num_segments,
+                        int64_t num_pairs, int64_t num_blocks, hipStream_t stream) {
+  const size_t pair_offset = copy_pair_offset(num_segments);
+  const CopySeg* segs = reinterpret_cast<const CopySeg*>(src);
+  const PairDesc* pairs = reinterpret_cast<const PairDesc*>(src + pair_offset);
   FillArgs a;
+  a.wide = num_blocks > (int64_t(1) << 32);
   a.pad = 0;
-  for (size_t off = 0; off < bytes; off += kFillBytes) {
-    const size_t n = std::min<size_t>(kFillBytes, bytes - off);
-    std::memcpy(a.data, src + off, n);
-    a.dst = reinterpret_cast<v4u*>(dst + off);
-    a.words = static_cast<uint32_t>(n / 16);
+  const size_t pair_bytes = a.wide ? sizeof(PairDesc) : sizeof(FillPair);
+  int64_t s = 0, p = 0;
+  while (s < num_segments || p < num_pairs) {
+    a.segs = reinterpret_cast<CopySeg*>(dst) + s;
+    a.pairs = reinterpret_cast<PairDesc*>(dst + pair_offset) + p;
+    a.num_segs = static_cast<uint32_t>(
+        std::min<int64_t>(num_segments - s, kFillBytes / sizeof(FillSeg)));
+    const size_t used = a.num_segs * sizeof(FillSeg);
+    a.num_pairs = static_cast<uint32_t>(
+        std::min<int64_t>(num_pairs - p, static_cast<int64_t>((kFillBytes - used) / pair_bytes)));
+    FillSeg* fs = reinterpret_cast<FillSeg*>(a.data);
+    for (uint32_t i = 0; i < a.num_segs; ++i) fs[i] = FillSeg{segs[s + i].dst, segs[s + i].page_bytes};
+    if (a.wide) {
+      std::memcpy(a.data + used, pairs + p, a.num_pairs * pair_bytes);
+    } else {
+      FillPair* fp = reinterpret_cast<FillPair*>(a.data + used);
+      for (uint32_t i = 0; i < a.num_pairs; ++i)
+        fp[i] = FillPair{static_cast<uint32_t>(pairs[p + i].src),
+                         static_cast<uint32_t>(pairs[p + i].dst)};
+    }
+    s += a.num_segs;
+    p += a.num_pairs;
     (void)hipGetLastError();  // clear a stale error: the check below is for this launch
-    hipLaunchKernelGGL(desc_fill_kernel, dim3(1), dim3(kFillBytes / 16), 0, stream, a);
+    hipLaunchKernelGGL(desc_fill_kernel, dim3(1), dim3(kFillLanes), 0, stream, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
@@ -2098,13 +2246,17 @@ int copy_noalloc(int32_t num_segments, void* const* bases, const int64_t* page_b
   if (!stream_has_all_cus(stream, num_cus))
     rc = copy_plan(t, vec, max_page, false, num_segments, num_pairs, &plan);
   if (rc) return rc;
-  pack_copy_desc(reinterpret_cast<char*>(g_noalloc_host), num_segments, bases, bases,
-                 page_bytes, num_pairs, src_ids, dst_ids, t.copy_order, g_noalloc_order);
-  const size_t total = copy_pair_offset(num_segments) + sizeof(PairDesc) * num_pairs;
+  bool launched = false;
+  rc = copy_inline(plan, t, num_cus, num_segments, bases, bases, page_bytes, num_pairs, src_ids,
+                   dst_ids, stream, &launched);
+  if (rc || launched) return rc;
+  pack_copy_desc(reinterpret_cast<char*>(g_noalloc_host), copy_pair_offset(num_segments),
+                 num_segments, bases, bases, page_bytes, num_pairs, src_ids, dst_ids,
+                 t.copy_order, g_noalloc_order);
   // The descriptor reaches `scratch` through kernel arguments, not a copy
   // from the packing area: a copy node captured into a graph would read the
   // packing area again at every replay, after later calls rewrote it.
-  hipError_t e = noalloc_fill(dv, g_noalloc_host, total, stream);
+  hipError_t e = noalloc_fill(dv, g_noalloc_host, num_segments, num_pairs, num_blocks, stream);
   if (e != hipSuccess) return hip_fail(e, "desc_fill_kernel launch");
   e = copy_launch(plan, t, num_cus, num_segments, dv, stream);
   if (e != hipSuccess) return hip_fail(e, "copy_blocks_kernel launch");

@@ -233,11 +233,12 @@ int aegkv_copy_blocks(int32_t num_segments, void* const* segment_bases,
  * the host or the device: the descriptor goes to a fixed device array of
  * 1,081,344 bytes that each GPU the library runs on holds until the process
  * ends, written there by small fill kernels whose arguments carry the
- * descriptor (2 KiB per launch; 4096 pairs over 80 segments take 34
- * launches). A graph that captures the call therefore replays the
+ * descriptor (3776 bytes per launch, 8 a pair; 4096 pairs over 80 segments
+ * take 10 launches), or, for a short call (94 pairs over 72 segments), in
+ * the arguments of the copy itself. A graph that captures the call therefore replays the
  * descriptor it captured, whatever calls ran since. The launches cost host
- * time: measured 0.48 ms per call for 4096 pairs over 80 segments and
- * 7.0 ms for 65536 pairs, against 0.10-0.11 ms for aegkv_copy_blocks; the
+ * time: measured 0.33 ms per call for 4096 pairs over 80 segments and
+ * 6.1 ms for 65536 pairs, against 0.05 and 0.41 ms for aegkv_copy_blocks; the
  * same for up to a few hundred pairs. Limits: at most 1024
  * segments and 65536 pairs per call (AEGKV_ENOMEM beyond, nothing
  * enqueued). Every call on a device shares that device's array, which keeps

@@ -127,3 +127,77 @@ def test_copy_blocks_noalloc_under_graph_capture(gpu):
         for i in range(n_seg):
             assert torch.equal(a[i], want[i]), (r, i)
     del graph
+
+
+# Descriptors around what one launch's arguments hold: the copy's own 3808
+# bytes (32 a segment, 16 a pair) and a fill's 3776 (16 a segment, 8 a pair).
+@pytest.mark.parametrize("page", [32, 33])
+@pytest.mark.parametrize("n_seg,n", [
+    (1, 235), (1, 236), (1, 237), (72, 94), (72, 95), (118, 2), (118, 3), (119, 1),
+    (1, 470), (1, 471), (1, 942), (1, 943), (236, 5), (237, 5), (237, 471),
+])
+def test_copies_with_descriptors_around_a_launch_s_arguments(gpu, n_seg, n, page):
+    _say("descriptors around a launch's arguments", n_seg, n, page)
+    rng = np.random.default_rng(n_seg * 1000 + n)
+    n_blocks = 2 * n + 3
+    a, _ = _caches(n_seg, n_blocks, page, n, gpu)
+    src, dst = _pairs(rng, n_blocks, n)
+    s, d = torch.from_numpy(src.copy()).to(gpu), torch.from_numpy(dst.copy()).to(gpu)
+    want = [t.clone().index_copy_(0, d, t[s]) for t in a]
+    for entry in (ops.copy_blocks, ops.copy_blocks_noalloc):
+        got = [t.clone() for t in a]
+        entry(got, src, dst)
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(got, want)), entry.__name__
+    other = [torch.zeros_like(t) for t in a]
+    ops.migrate_blocks(a, other, src, dst)
+    torch.cuda.synchronize()
+    for t, o, w in zip(a, other, want):
+        assert torch.equal(o[d], w[d]) and int((o != 0).any(1).sum()) <= n
+
+
+@pytest.mark.parametrize("n", [3, 250, 400])
+def test_block_ids_beyond_32_bits(gpu, n):
+    """A cache of more blocks than 32-bit ids name (1-byte pages): the copy
+    with its descriptor in the launch, and one and two fill launches of
+    whole 16-byte pairs."""
+    _say("block ids beyond 32 bits", n)
+    n_blocks = (1 << 32) + 1000
+    a = torch.zeros(n_blocks, 1, dtype=torch.uint8, device=gpu)
+    rng = np.random.default_rng(n)
+    ids = rng.permutation(1000)
+    src, dst = ids[:n] + (1 << 32) - 500, ids[n:2 * n] + (1 << 32) - 500
+    s, d = torch.from_numpy(src).to(gpu), torch.from_numpy(dst).to(gpu)
+    a[s] = torch.randint(1, 256, (n, 1), dtype=torch.uint8, device=gpu)
+    ops.copy_blocks_noalloc([a], src, dst)
+    torch.cuda.synchronize()
+    assert torch.equal(a[d], a[s])
+    assert not a[:4096].any() and int((a[-2000:] != 0).sum()) == 2 * n
+
+
+@pytest.mark.parametrize("n", [20, 600])
+def test_short_and_long_captured_copies_replay_their_own_pairs(gpu, n):
+    """As above for a descriptor inside the copy's own launch and for one of
+    two fill launches, with both kinds of eager call between the replays."""
+    _say("captured copies", n)
+    rng = np.random.default_rng(n)
+    a, _ = _caches(6, 2048, 4096, n, gpu)
+    perm = rng.permutation(2048)
+    sa, da, rest = perm[:n], perm[n:2 * n], perm[2 * n:]
+    ia, ja = torch.from_numpy(sa.copy()).to(gpu), torch.from_numpy(da.copy()).to(gpu)
+    ops.copy_blocks_noalloc(a, rest[:1], rest[1:2])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream(gpu)):
+        ops.copy_blocks_noalloc(a, sa, da)
+    for r in range(4):
+        for t in a:
+            t[ja] = r + 1
+        ops.copy_blocks_noalloc(a, rest[:5 + r], rest[10:15 + r])
+        ops.copy_blocks_noalloc(a, rest[20:420], rest[420:820])
+        torch.cuda.synchronize()
+        want = [t.clone().index_copy_(0, ja, t[ia]) for t in a]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(a, want)), r
+    del graph
