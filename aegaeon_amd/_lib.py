@@ -94,6 +94,9 @@ _I32P = ctypes.POINTER(ctypes.c_int32)
 _U64P = ctypes.POINTER(ctypes.c_uint64)
 _PP = ctypes.POINTER(ctypes.c_void_p)
 
+# Tables and id lists of the moves are taken as plain addresses, so that the
+# packed bytes of _hostargs go through as they are (ctypes passes a bytes
+# object's own buffer and holds it for the call) beside ctypes pointers.
 _SIGNATURES = {
     "aegkv_abi_version": (_INT, []),
     "aegkv_init": (_INT, []),
@@ -103,14 +106,13 @@ _SIGNATURES = {
     "aegkv_swap_blocks": (
         _INT,
         [_I32, _PP, _I64P, _I64P, _U64P, _I64, _I32, _I64P, _P, _I64, _I64, _I64, _I64,
-         _I64P, _I64P, _I32P, _I64P, _I64P, _INT, _INT, _P, _P],
+         _P, _P, _P, _P, _P, _INT, _INT, _P, _P],
     ),
-    "aegkv_copy_blocks": (_INT, [_I32, _PP, _I64P, _I64, _I64, _I64P, _I64P, _P]),
-    "aegkv_copy_blocks_noalloc": (_INT, [_I32, _PP, _I64P, _I64, _I64, _I64P, _I64P, _P]),
-    "aegkv_copy_probe": (_INT, [_INT, _I32, _PP, _I64P, _I64, _I64, _I64P, _I64P, _P,
+    "aegkv_copy_blocks": (_INT, [_I32, _P, _P, _I64, _I64, _P, _P, _P]),
+    "aegkv_copy_blocks_noalloc": (_INT, [_I32, _P, _P, _I64, _I64, _P, _P, _P]),
+    "aegkv_copy_probe": (_INT, [_INT, _I32, _P, _P, _I64, _I64, _P, _P, _P,
                                 ctypes.c_uint32, _P]),
-    "aegkv_migrate_blocks": (_INT, [_I32, _PP, _PP, _I64P, _I64, _I64, _I64, _I64P, _I64P, _P,
-                                    _P]),
+    "aegkv_migrate_blocks": (_INT, [_I32, _P, _P, _P, _I64, _I64, _I64, _P, _P, _P, _P]),
     "aegkv_load_slices": (_INT, [_I64, _PP, _PP, _I64P, _INT, _P]),
     "aegkv_transfer_entries": (
         _INT,
@@ -181,6 +183,23 @@ def load(path: str | os.PathLike | None = None) -> ctypes.CDLL:
                 raise AegkvError(rc, lib.aegkv_last_error().decode(errors="replace"))
         _lib = lib
         return lib
+
+
+_hostargs = None
+
+
+def hostargs():
+    """The native argument readers (csrc/hostargs.cpp), loaded once."""
+    global _hostargs
+    if _hostargs is None:
+        try:
+            from . import _hostargs as module
+        except ImportError as exc:
+            raise ImportError("aegaeon_amd/_hostargs.so is missing or does not fit this torch: "
+                              "build the library first "
+                              "(python -c 'import __graft_entry__ as g; g.build()')") from exc
+        _hostargs = module
+    return _hostargs
 
 
 def check(status: int) -> None:

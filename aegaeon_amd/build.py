@@ -1,4 +1,4 @@
-"""Build libaegkv.so (HIP, gfx950) in-tree with hipcc.
+"""Build libaegkv.so (HIP, gfx950, with hipcc) and _hostargs.so (host C++) in-tree.
 
 The library is a plain C-ABI shared object; it links against the HIP
 runtime by SONAME (libamdhip64.so.7), so inside a process that has already
@@ -10,12 +10,14 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 REPO_DIR = PKG_DIR.parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libaegkv.so"
+HOSTARGS_PATH = PKG_DIR / "_hostargs.so"
 ARCH = os.environ.get("AEGKV_OFFLOAD_ARCH", "gfx950")
 
 HIPCC_FLAGS = [
@@ -38,9 +40,35 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found: the HIP toolchain is required to build libaegkv")
 
 
+def build_hostargs(verbose: bool = False) -> Path:
+    """Compile csrc/hostargs.cpp into aegaeon_amd/_hostargs.so (always
+    rebuilds): a Python module over torch's C++ interface."""
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    tmp = HOSTARGS_PATH.with_suffix(".so.tmp")
+    cmd = [
+        os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        *[f"-isystem{p}" for p in (*include_paths(), sysconfig.get_paths()["include"])],
+        str(CSRC / "hostargs.cpp"),
+        *[f"-L{p}" for p in library_paths()],
+        "-ltorch_python", "-ltorch_cpu", "-lc10",
+        "-o", str(tmp),
+    ]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed ({res.returncode}):\n{res.stderr}")
+    os.replace(tmp, HOSTARGS_PATH)
+    return HOSTARGS_PATH
+
+
 def build(verbose: bool = False) -> Path:
     """Compile csrc/aegkv.hip, csrc/fence.hip and csrc/plan.cpp into
-    aegaeon_amd/libaegkv.so (always rebuilds)."""
+    aegaeon_amd/libaegkv.so, and csrc/hostargs.cpp (always rebuilds)."""
+    build_hostargs(verbose)
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [
         hipcc(),

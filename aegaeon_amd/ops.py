@@ -63,6 +63,25 @@ def _i32(values) -> np.ndarray:
     return np.ascontiguousarray(a.astype(np.int32, copy=False))
 
 
+def _id_arg(values):
+    """(C argument, count) of an id list: packed in one native pass where it
+    is a list of Python integers, as planners make it, else through _i64."""
+    packed = _lib.hostargs().pack_ids(values)
+    if packed is not None:
+        return packed, len(packed) // 8
+    a = _i64(values)
+    return _p64(a), a.size   # the pointer keeps the array
+
+
+def _group_arg(values):
+    """_id_arg for 32-bit group ids."""
+    packed = _lib.hostargs().pack_ids32(values, 1 << 31)
+    if packed is not None:
+        return packed, len(packed) // 4
+    a = _i32(values)
+    return _p32(a), a.size
+
+
 def _p64(a: np.ndarray):
     return a.ctypes.data_as(ctypes.POINTER(ctypes.c_int64))
 
@@ -76,8 +95,12 @@ def _pu64(a: np.ndarray):
 
 
 def _stream_ptr(device: torch.device, stream: torch.cuda.Stream | None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream(device)
-    return s.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if device.index is not None and torch.cuda.is_initialized():
+        # the same stream without making a Stream object of it (2.6 us)
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def _tensor_bytes(t: torch.Tensor) -> int:
@@ -223,22 +246,22 @@ class SegmentLayout:
         """One aegkv_swap_blocks call over this layout (see swap_segments).
         guard (with guard_index): a move guard word (GuardWords.tensor); when
         it is set by the time the stream reaches the swap, nothing moves."""
-        src = _i64(source_block_ids)
-        dst = _i64(target_block_ids)
-        grp = _i32(group_ids)
-        first = _i64(first_kernel_blocks)
-        valid = _i64(valid_kernel_blocks)
-        if not (src.size == dst.size == grp.size == first.size == valid.size):
+        self._swap_packed(_id_arg(source_block_ids), _id_arg(target_block_ids),
+                          _group_arg(group_ids), _id_arg(first_kernel_blocks),
+                          _id_arg(valid_kernel_blocks), is_swap_in, mode, stream,
+                          _guard_ptr(guard, guard_index, "guard"))
+
+    def _swap_packed(self, src, dst, grp, first, valid, is_swap_in, mode, stream, guard):
+        """swap() with its lists as (C argument, count)."""
+        if not (src[1] == dst[1] == grp[1] == first[1] == valid[1]):
             raise ValueError(
-                f"swap lists of unequal lengths: {src.size} sources, {dst.size} targets, "
-                f"{grp.size} groups, {first.size} first and {valid.size} valid kernel blocks"
+                f"swap lists of unequal lengths: {src[1]} sources, {dst[1]} targets, "
+                f"{grp[1]} groups, {first[1]} first and {valid[1]} valid kernel blocks"
             )
-        gp = _guard_ptr(guard, guard_index, "guard")
         lib = _lib.load()
         rc = _call_on(self.device, lambda: lib.aegkv_swap_blocks(
-            *self._args, src.size, _p64(src), _p64(dst), _p32(grp), _p64(first),
-            _p64(valid), 1 if is_swap_in else 0, _mode(mode), gp,
-            _stream_ptr(self.device, stream)))
+            *self._args, src[1], src[0], dst[0], grp[0], first[0], valid[0],
+            1 if is_swap_in else 0, _mode(mode), guard, _stream_ptr(self.device, stream)))
         _lib.check(rc)
 
 
@@ -281,8 +304,18 @@ def swap_segments(
 
 def _copy_call_args(segments, src_block_ids, dst_block_ids, segment_page_bytes,
                     device_num_blocks, stream):
-    """Checked C-ABI arguments of one copy_blocks call (device first; the
-    arrays are returned too so they outlive the call)."""
+    """Checked C-ABI arguments of one copy_blocks call (device first)."""
+    if segment_page_bytes is None:
+        table = _lib.hostargs().segment_table(segments, device_num_blocks)
+        if table is not None:
+            _, blocks, bases, page = table
+            src, n = _id_arg(src_block_ids)
+            dst, n_dst = _id_arg(dst_block_ids)
+            if n != n_dst:
+                raise ValueError("src and dst id lists differ in length")
+            dev = segments[0].device
+            return dev, (len(bases) // 8, bases, page, blocks, n, src, dst,
+                         _stream_ptr(dev, stream))
     if not segments:
         raise ValueError("at least one segment is required")
     dev = segments[0].device
@@ -307,7 +340,7 @@ def _copy_call_args(segments, src_block_ids, dst_block_ids, segment_page_bytes,
     bases = (ctypes.c_void_p * len(segments))(*[t.data_ptr() for t in segments])
     args = (len(segments), bases, _p64(page), int(device_num_blocks), src.size, _p64(src),
             _p64(dst), _stream_ptr(dev, stream))
-    return dev, args, (page, src, dst)
+    return dev, args   # the pointers keep their arrays
 
 
 def copy_blocks(
@@ -326,8 +359,8 @@ def copy_blocks(
     from the sources. The reference has no KV copy_blocks; its in-HBM
     compaction is aegaeon/allocator.py:101-137.
     """
-    dev, args, _keep = _copy_call_args(segments, src_block_ids, dst_block_ids,
-                                       segment_page_bytes, device_num_blocks, stream)
+    dev, args = _copy_call_args(segments, src_block_ids, dst_block_ids,
+                                segment_page_bytes, device_num_blocks, stream)
     lib = _lib.load()
     _lib.check(_call_on(dev, lambda: lib.aegkv_copy_blocks(*args)))
 
@@ -350,8 +383,8 @@ def copy_probe(kind: int, segments: Sequence[torch.Tensor], src_block_ids, dst_b
         raise ValueError(f"unknown probe kind {kind!r}")
     if sink.device.type != "cuda" or sink.element_size() != 4 or sink.numel() < 1:
         raise ValueError("sink must be a device tensor of 4-byte words")
-    dev, args, _keep = _copy_call_args(segments, src_block_ids, dst_block_ids,
-                                       segment_page_bytes, device_num_blocks, stream)
+    dev, args = _copy_call_args(segments, src_block_ids, dst_block_ids,
+                                segment_page_bytes, device_num_blocks, stream)
     lib = _lib.load()
     _lib.check(_call_on(dev, lambda: lib.aegkv_copy_probe(
         kind, *args[:-1], sink.data_ptr(), int(magic) & 0xFFFFFFFF, args[-1])))
@@ -377,8 +410,8 @@ def copy_blocks_noalloc(
     NOALLOC_MAX_PAIRS pairs (ValueError beyond). Calls that overlap on one
     device from different streams or threads race on that array; calls on
     one stream are ordered."""
-    dev, args, _keep = _copy_call_args(segments, src_block_ids, dst_block_ids,
-                                       segment_page_bytes, device_num_blocks, stream)
+    dev, args = _copy_call_args(segments, src_block_ids, dst_block_ids,
+                                segment_page_bytes, device_num_blocks, stream)
     lib = _lib.load()
     _lib.check(_call_on(dev, lambda: lib.aegkv_copy_blocks_noalloc(*args)))
 
@@ -442,6 +475,21 @@ def migrate_blocks(
     """
     if not src_segments or len(src_segments) != len(dst_segments):
         raise ValueError("one source and one target tensor per segment are required")
+    if segment_page_bytes is None:
+        table = _lib.hostargs().segment_table
+        st, dt = table(src_segments, None), table(dst_segments, None)
+        if st is not None and dt is not None and st[3] == dt[3]:
+            src, n = _id_arg(src_block_ids)
+            dst, n_ids = _id_arg(dst_block_ids)
+            if n != n_ids:
+                raise ValueError("src and dst id lists differ in length")
+            gp = _guard_ptr(guard, guard_index, "guard")
+            dev = dst_segments[0].device
+            lib = _lib.load()
+            _lib.check(_call_on(dev, lambda: lib.aegkv_migrate_blocks(
+                len(dt[2]) // 8, st[2], dt[2], dt[3], st[1], dt[1], n, src, dst, gp,
+                _stream_ptr(dev, stream))))
+            return
     dev = dst_segments[0].device
     for i, (a, b) in enumerate(zip(src_segments, dst_segments)):
         _require_device(a, f"source segment {i}")

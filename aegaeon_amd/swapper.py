@@ -49,7 +49,7 @@ from typing import Dict, List, Optional, Sequence, Tuple, Union
 import numpy as np
 import torch
 
-from . import ops
+from . import _lib, ops
 from .cache_groups import CacheGroupRuntimeConfig
 from .layout import CompositeCache, host_page_geometry
 
@@ -355,11 +355,17 @@ class KVSwapper:
                 "kernel blocks"
             )
         self._require_open()
-        groups = np.asarray(group_ids, dtype=np.int64).reshape(-1)
-        if groups.size and (groups.min() < 0 or groups.max() >= len(self.group_descriptors)):
-            bad = groups[(groups < 0) | (groups >= len(self.group_descriptors))][0]
-            raise ValueError(f"cache-group id {int(bad)} of a swap entry is not one of the "
-                             f"{len(self.group_descriptors)} groups")
+        # a list of known groups is packed as it is; anything else is looked at
+        packed = _lib.hostargs().pack_ids32(group_ids, len(self.group_descriptors))
+        if packed is not None:
+            grp = packed, len(packed) // 4
+        else:
+            groups = np.asarray(group_ids, dtype=np.int64).reshape(-1)
+            if groups.size and (groups.min() < 0 or groups.max() >= len(self.group_descriptors)):
+                bad = groups[(groups < 0) | (groups >= len(self.group_descriptors))][0]
+                raise ValueError(f"cache-group id {int(bad)} of a swap entry is not one of the "
+                                 f"{len(self.group_descriptors)} groups")
+            grp = ops._group_arg(groups.astype(np.int32))
         side = 1 if is_swap_in else 0
         self._require_not_failed(side)
         stream = self.swap_in_stream if is_swap_in else self.swap_out_stream
@@ -367,12 +373,13 @@ class KVSwapper:
         # wait for in-flight moves of the same requests (worker.py:2351-2394);
         # bytes are IPC handles exported by another process
         self._wait_sources(request_ids, source_events, stream, side)
-        self._layout.swap(source_block_ids, target_block_ids, groups.astype(np.int32),
-                          first_kernel_blocks, valid_kernel_blocks, is_swap_in,
-                          mode=self.mode if mode is None else mode, stream=stream,
-                          guard=self.guards.tensor, guard_index=side)
+        self._layout._swap_packed(
+            ops._id_arg(source_block_ids), ops._id_arg(target_block_ids), grp,
+            ops._id_arg(first_kernel_blocks), ops._id_arg(valid_kernel_blocks), is_swap_in,
+            self.mode if mode is None else mode, stream, self.guards.ptr(side))
         self._finish(request_ids, side, stream, new_event)
         if logger.isEnabledFor(logging.INFO):
+            groups = np.asarray(group_ids, dtype=np.int64).reshape(-1)
             valid = np.asarray(valid_kernel_blocks, dtype=np.int64).reshape(-1)
             copied = int((valid * self._bytes_per_kb[groups]).sum()) if groups.size else 0
             extents = int(((valid > 0) * self._extents_per_entry[groups]).sum()) if groups.size else 0

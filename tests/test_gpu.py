@@ -404,6 +404,55 @@ def test_copy_on_a_masked_stream_vs_expectation(gpu, page):
         masked.close()
 
 
+class _Sub(torch.Tensor):
+    pass
+
+
+def test_segment_table_reads_what_the_general_path_reads(gpu):
+    """Plain device tensors give one native table; every other kind of
+    argument is left to the general path, with its results and refusals."""
+    from aegaeon_amd import _lib
+
+    table = _lib.hostargs().segment_table
+    a = [torch.zeros(6, 3 + i, dtype=d, device=gpu) for i, d in
+         enumerate((torch.uint8, torch.bfloat16, torch.float32))]
+    for segs, blocks in ((a, None), (tuple(a), None), (a, 3), (a[:1], 1), (a, 4)):
+        index, n, bases, pages = table(segs, blocks)
+        assert index == a[0].get_device() and n == (blocks or 6)
+        assert np.frombuffer(bases, np.int64).tolist() == [t.data_ptr() for t in segs]
+        assert np.frombuffer(pages, np.int64).tolist() == [
+            t.numel() * t.element_size() // n for t in segs]
+    scalar = torch.zeros((), device=gpu)
+    for segs, blocks in ((a, 0), (a, -1), (a, 2.0), (a, np.int64(3)), (a, True),
+                         ([a[0], a[1].t()], None), ([a[0], torch.zeros(6, 4)], None),
+                         ([a[2].as_subclass(_Sub)], None), ([scalar], None),
+                         ([torch.zeros(0, 4, device=gpu)], None), (iter(a), None)):
+        assert table(segs, blocks) is None, (segs, blocks)
+    with pytest.raises(ValueError, match="contiguous"):
+        ops.copy_blocks([a[0], a[1].t()], [0], [1])
+    with pytest.raises(ValueError, match="differ in length"):
+        ops.copy_blocks(a, [0, 1], [2])
+    with pytest.raises(ValueError, match="integers"):
+        ops.copy_blocks(a, [0.0], [1.0])
+    # the same copy through every kind of list and through given pages
+    ids = ([0, 2], [1, 5])
+    a[0].random_(), a[2].random_()
+    want = [t.clone() for t in a]
+    for w in want:
+        w[1], w[5] = w[0].clone(), w[2].clone()
+    for kind in (list, tuple, np.array, torch.tensor):
+        for pages in (None, [t.numel() * t.element_size() // 6 for t in a]):
+            got = [t.clone() for t in a]
+            ops.copy_blocks(got, kind(ids[0]), kind(ids[1]), segment_page_bytes=pages)
+            torch.cuda.synchronize()
+            assert all(torch.equal(x, y) for x, y in zip(got, want)), (kind, pages)
+    for wrap in (torch.nn.Parameter, lambda t: t.as_subclass(_Sub)):
+        got = [t.clone() for t in a[1:]]
+        ops.copy_blocks([wrap(t) for t in got], *ids)
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(got, want[1:]))
+
+
 def _shifted(nbytes, shift, device, g):
     """Random device bytes starting `shift` bytes behind a 16-byte boundary,
     with 64 bytes around them that no move may touch: (all, the view)."""

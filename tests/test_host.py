@@ -874,3 +874,58 @@ def test_launch_item_bound_before_any_hip_call(aegkv_lib):
         assert rc == _lib.EINVAL
         msg = lib.aegkv_last_error()
         assert (b"work items of one launch" in msg) == refused, msg
+
+
+@pytest.mark.parametrize("values", [
+    [], [0], [5, -1, 2 ** 62], (7, 8), list(range(1000)), [2 ** 63 - 1, -2 ** 63],
+    [2 ** 63], [1.0], [True], [np.int64(3)], np.arange(4), np.arange(4, dtype=np.int32),
+    torch.tensor([1, 2]), range(5), [[1, 2], [3, 4]], "12", b"12", [None],
+])
+def test_packed_ids_equal_the_general_conversion(aegkv_lib, values):
+    """A list of Python integers is packed natively; whatever is not one gives
+    what the general conversion gives, its refusals included."""
+    from aegaeon_amd import _lib, ops
+
+    def outcome(fn):
+        try:
+            return fn()
+        except (ValueError, OverflowError, TypeError) as exc:
+            return type(exc)
+
+    def through_arg():
+        arg, n = ops._id_arg(values)
+        if not isinstance(arg, bytes):
+            return [arg[i] for i in range(n)]
+        assert len(arg) == 8 * n
+        return np.frombuffer(arg, np.int64).tolist()
+
+    assert outcome(through_arg) == outcome(lambda: ops._i64(values).tolist())
+    packed = _lib.hostargs().pack_ids(values)
+    plain = isinstance(values, (list, tuple)) and all(
+        type(v) is int and -2 ** 63 <= v < 2 ** 63 for v in values)
+    assert (packed is not None) == plain
+
+
+@pytest.mark.parametrize("values,limit", [
+    ([], 1), ([0, 1, 0], 2), ([0, 2], 2), ([-1], 2), ([2 ** 31 - 1], 2 ** 31), ([2 ** 31], 2 ** 40),
+    ([True], 2), ([0.0], 2), (np.zeros(2, np.int32), 2), ((1,), 2),
+])
+def test_packed_group_ids(aegkv_lib, values, limit):
+    from aegaeon_amd import _lib
+
+    packed = _lib.hostargs().pack_ids32(values, limit)
+    plain = isinstance(values, (list, tuple)) and all(
+        type(v) is int and 0 <= v < min(limit, 2 ** 31) for v in values)
+    assert (packed is not None) == plain
+    if plain:
+        assert np.frombuffer(packed, np.int32).tolist() == list(values)
+
+
+def test_segment_table_leaves_host_tensors_to_the_general_path(aegkv_lib):
+    from aegaeon_amd import _lib, ops
+
+    table = _lib.hostargs().segment_table
+    for segs in ([torch.zeros(4, 8)], [], [3], torch.zeros(2, 4, 8), [torch.zeros(4, 8).t()]):
+        assert table(segs, None) is None
+    with pytest.raises(ValueError, match="device"):
+        ops.copy_blocks([torch.zeros(4, 8)], [0], [1])
