@@ -48,6 +48,7 @@ TUNE_STAGED_OVERLAP = 14
 TUNE_SWAP_OUT_WORKGROUPS_UNCACHED = 15
 TUNE_COPY_LANES = 17
 TUNE_COPY_ORDER = 18
+TUNE_STAGED_SHORT_RUNS = 19
 HOST_UNCACHED = 1
 HOST_COHERENT = 2
 PROBE_READ = 1

@@ -113,6 +113,7 @@ struct Tunables {
   // swap-out's copies to SDMA and it fell to 29 GB/s (35 one chunk at a
   // time); set bit 0 off for that pattern.
   int64_t staged_overlap = 3;
+  int64_t staged_short_runs = 1;  // STAGED calls of short runs go DIRECT (runs_are_short)
   // copy_blocks, 1024-lane shapes with items of >= 32 KiB (a fixed unroll):
   // LDS reserved per workgroup so that one workgroup holds a CU (HBM copy
   // rate +1-5 % on 32-160 KiB tiles).
@@ -1491,6 +1492,38 @@ void entry_runs(const SwapLayout& L, const SwapList& E, int64_t i, bool is_swap_
   }
 }
 
+// The runs of a staged chunk, order[lo, hi), in staging slots of their own.
+void chunk_runs(const SwapLayout& L, const SwapList& E, const std::vector<int64_t>& order,
+                size_t lo, size_t hi, bool is_swap_in, int64_t composite,
+                std::vector<Run>& runs) {
+  runs.clear();
+  for (size_t j = lo; j < hi; ++j)
+    entry_runs(L, E, order[j], is_swap_in, static_cast<int64_t>(j - lo), composite, runs);
+}
+
+// How a STAGED call's runs move, by the runs of its first chunk.
+//
+// The runtime takes 3-7 us a copy, over two streams, so runs below 128 KiB on
+// average stay under a third of the link rate: such calls go out as the
+// DIRECT kernel. 480 runs of 9 KiB: 1315 us staged, 81 direct; 60 blocks of
+// 40 KiB, some adjacent: 229 and 47. Longer runs stay staged, which leaves
+// the CUs alone.
+//
+// Up to four runs in one chunk leave nothing to overlap, so their copies go
+// on the caller's stream, without the events that fork to the library's
+// streams and back (20-40 us): one run of 9.4 MB 265 -> 225 us, of 47 MB 942
+// -> 907, of 2.5 MB 166 -> 103, and with several callers in turn, where the
+// runtime moves some copies at 29 GB/s, of 472 MB 10.4 -> 9.15 ms. Four runs
+// of 2.4 MB 272 -> 254 us, twenty 1002 -> 1058.
+constexpr int64_t kShortRun = int64_t(128) << 10;
+constexpr size_t kFewRuns = 4;
+
+bool runs_are_short(const std::vector<Run>& runs) {
+  int64_t bytes = 0;
+  for (const Run& r : runs) bytes += r.len;
+  return runs.size() > kFewRuns && bytes < kShortRun * static_cast<int64_t>(runs.size());
+}
+
 // A stream on a hardware queue of its own: a stream created with a CU mask
 // gets a dedicated queue (here the mask enables every CU), while plain
 // streams share the process's GPU_MAX_HW_QUEUES queues, and two copies whose
@@ -1598,16 +1631,15 @@ int chunk_copies(DeviceCtx* ctx, int k, const std::vector<Run>& runs, bool to_de
 
 // STAGED one chunk after another, each through its own stream-ordered
 // staging allocation: swap-out gathers a chunk and then copies it to the
-// host, swap-in copies a chunk from the host and then scatters it.
+// host, swap-in copies a chunk from the host and then scatters it. `runs`
+// arrives with those of the first chunk.
 int staged_serial(DeviceCtx* ctx, const SwapLayout& L, const SwapList& E,
                   const std::vector<int64_t>& order, bool is_swap_in, int64_t composite,
-                  size_t step, bool vec_stage, const Tunables& t, int k, hipStream_t stream) {
-  std::vector<Run> runs;
+                  size_t step, std::vector<Run>& runs, bool vec_stage, const Tunables& t, int k,
+                  hipStream_t stream) {
   for (size_t lo = 0; lo < order.size(); lo += step) {
     const size_t hi = std::min(order.size(), lo + step);
-    runs.clear();
-    for (size_t j = lo; j < hi; ++j)
-      entry_runs(L, E, order[j], is_swap_in, static_cast<int64_t>(j - lo), composite, runs);
+    if (lo > 0) chunk_runs(L, E, order, lo, hi, is_swap_in, composite, runs);
     void* p = nullptr;
     AEGKV_HIP(hipMallocAsync(&p, (hi - lo) * static_cast<size_t>(composite), stream));
     char* buf = static_cast<char*>(p);
@@ -1640,8 +1672,8 @@ int staged_serial(DeviceCtx* ctx, const SwapLayout& L, const SwapList& E,
 // and frees the buffers there.
 int staged_overlapped(DeviceCtx* ctx, const SwapLayout& L, const SwapList& E,
                       const std::vector<int64_t>& order, bool is_swap_in, int64_t composite,
-                      size_t step, bool vec_stage, const Tunables& t, int k,
-                      hipStream_t stream) {
+                      size_t step, std::vector<Run>& runs, bool vec_stage, const Tunables& t,
+                      int k, hipStream_t stream) {
   DeviceCtx::DmaSet& d = ctx->dma[is_swap_in ? 1 : 0];
   std::lock_guard<std::mutex> lk(d.mu);
   int rc = ensure_dma(d, k);
@@ -1685,13 +1717,10 @@ int staged_overlapped(DeviceCtx* ctx, const SwapLayout& L, const SwapList& E,
   };
   hipError_t e = fan_in(d.fork_ev, &d.fork_on, stream);
   if (e != hipSuccess) return unwind(hip_fail(e, "staged fork"));
-  std::vector<Run> runs;
   for (size_t c = 0; c < chunks; ++c) {
     const size_t lo = c * step, hi = std::min(n, lo + step);
     const int b = static_cast<int>(c & 1);
-    runs.clear();
-    for (size_t j = lo; j < hi; ++j)
-      entry_runs(L, E, order[j], is_swap_in, static_cast<int64_t>(j - lo), composite, runs);
+    if (c > 0) chunk_runs(L, E, order, lo, hi, is_swap_in, composite, runs);
     if (!is_swap_in) {
       if (c >= 2 && (e = join(b)) != hipSuccess)
         return unwind(hip_fail(e, "hipStreamWaitEvent(staged copies)"));
@@ -1761,7 +1790,7 @@ int swap_core(const SwapLayout& L, const SwapList& E, bool is_swap_in, int mode,
   std::vector<int64_t> order(static_cast<size_t>(E.n));
   for (int64_t i = 0; i < E.n; ++i) order[static_cast<size_t>(i)] = i;
 
-  if (!staged) {
+  auto direct = [&] {
     std::lock_guard<std::mutex> lk(ctx->mu);
     // link-bound: a few persistent workgroups
     const int64_t wgs = is_swap_in                        ? t.swap_in_workgroups
@@ -1770,7 +1799,8 @@ int swap_core(const SwapLayout& L, const SwapList& E, bool is_swap_in, int mode,
     return enqueue_swap_kernel(ctx, L, E, order, 0, order.size(), is_swap_in, false,
                                L.host_pool, L.host_page_bytes, L.host_rank_offset,
                                dev_vec && host_vec, wgs, stream);
-  }
+  };
+  if (!staged) return direct();
 
   // STAGED: host-id order lets consecutive host pages merge into one DMA.
   const int64_t* host_ids = is_swap_in ? E.src : E.dst;
@@ -1778,15 +1808,19 @@ int swap_core(const SwapLayout& L, const SwapList& E, bool is_swap_in, int mode,
                    [&](int64_t a, int64_t b) { return host_ids[a] < host_ids[b]; });
   const size_t step = static_cast<size_t>(
       std::max<int64_t>(1, std::min<int64_t>(E.n, t.staging_bytes / composite)));
+  std::vector<Run> runs;
+  chunk_runs(L, E, order, 0, step, is_swap_in, composite, runs);
+  if (t.staged_short_runs && runs_are_short(runs)) return direct();
   // Staging comes from hipMallocAsync (256 B aligned) with a composite stride.
   const bool vec_stage = dev_vec && composite % 16 == 0;
-  const int k = static_cast<int>(std::min<int64_t>(t.staged_dma_streams, kMaxDmaStreams));
+  int k = static_cast<int>(std::min<int64_t>(t.staged_dma_streams, kMaxDmaStreams));
+  if (order.size() <= step && runs.size() <= kFewRuns) k = 0;
   const bool overlap = (t.staged_overlap >> (is_swap_in ? 1 : 0)) & 1;
   if (k <= 1 || !overlap)
-    return staged_serial(ctx, L, E, order, is_swap_in, composite, step, vec_stage, t, k,
+    return staged_serial(ctx, L, E, order, is_swap_in, composite, step, runs, vec_stage, t, k,
                          stream);
-  return staged_overlapped(ctx, L, E, order, is_swap_in, composite, step, vec_stage, t, k,
-                           stream);
+  return staged_overlapped(ctx, L, E, order, is_swap_in, composite, step, runs, vec_stage, t,
+                           k, stream);
 }
 
 // Whole-block copies from a source cache to a target cache (the same cache
@@ -2382,6 +2416,7 @@ int64_t aegkv_tune(int key, int64_t value) {
     case AEGKV_TUNE_STAGED_OVERLAP: slot = &g_tune.staged_overlap; break;
     case AEGKV_TUNE_SWAP_OUT_WORKGROUPS_UNCACHED: slot = &g_tune.swap_out_workgroups_uncached; break;
     case AEGKV_TUNE_COPY_ORDER: slot = &g_tune.copy_order; break;
+    case AEGKV_TUNE_STAGED_SHORT_RUNS: slot = &g_tune.staged_short_runs; break;
     default: return fail(AEGKV_EINVAL, "unknown tuning key %d", key);
   }
   const int64_t prev = *slot;
@@ -2419,6 +2454,8 @@ int64_t aegkv_tune(int key, int64_t value) {
     if (key == AEGKV_TUNE_COPY_LDS_BYTES && value > kMaxLdsPerWorkgroup)
       return fail(AEGKV_EINVAL, "copy LDS reservation must be in [0, %lld]",
                   static_cast<long long>(kMaxLdsPerWorkgroup));
+    if (key == AEGKV_TUNE_STAGED_SHORT_RUNS && value > 1)
+      return fail(AEGKV_EINVAL, "tuning key %d takes 0 or 1", key);
     if (key == AEGKV_TUNE_SWAP_SHAPE_AUTO && value > 1)
       return fail(AEGKV_EINVAL, "swap shape selector is 0 or 1");
     if (key == AEGKV_TUNE_STAGED_OVERLAP && value > 3)
