@@ -341,32 +341,47 @@ __device__ __forceinline__ void move_any(const char* src, char* dst, uint32_t nb
   if (edge) ((gchar*)dst)[at] = b;
 }
 
+// A guard in the caller's own place, pinned host memory perhaps: one lane of
+// each workgroup reads it (83 ns a read, one after another: for grids of a
+// few workgroups). Every lane of the workgroup gets the same answer.
+__device__ __forceinline__ bool guard_set_at_source(const uint64_t* guard) {
+  if (guard == nullptr) return false;
+  __shared__ uint32_t set;
+  if (threadIdx.x == 0)
+    set = __hip_atomic_load(guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0;
+  __syncthreads();
+  return set != 0;
+}
+
+// What a swap kernel needs beside its tables.
+struct SwapWalk {
+  char* host_base;
+  int64_t host_stride, host_rank_offset;
+  uint32_t num_segs, num_items, chunks_per_tile;
+};
+
 // Swap tile mover. Item w -> (entry e, segment s, chunk c), entry-major.
 // TO_HOST: device tile -> host side; otherwise host side -> device tile.
-// The host keeps num_items + gridDim.x below 2^32 (items_fit_launch), so the
+// The host keeps num_items + gridDim.x below 2^32 (launch_items), so the
 // 32-bit grid-stride loop never wraps.
-template <int WG, int U, bool TO_HOST, bool VEC, bool NT_STORE>
-__global__ __launch_bounds__(WG) void swap_tiles_kernel(
-    const SegDesc* __restrict__ segs, const EntDesc* __restrict__ ents,
-    const int64_t* __restrict__ kpp, uint32_t num_segs, uint32_t num_items,
-    uint32_t chunks_per_tile, char* host_base, int64_t host_stride, int64_t host_rank_offset,
-    const uint64_t* guard) {
+template <int WG, int U, bool TO_HOST, bool VEC, bool NT_STORE, typename Segs, typename Ents,
+          typename Kpp>
+__device__ __forceinline__ void swap_items(Segs segs, Ents ents, Kpp kpp, const SwapWalk& k) {
   constexpr int64_t kChunk = Shape<WG, U>::kChunk;
-  if (guard_set(guard)) return;
-  for (uint32_t w = blockIdx.x; w < num_items; w += gridDim.x) {
-    const uint32_t tile = w / chunks_per_tile;
-    const uint32_t c = w - tile * chunks_per_tile;
-    const uint32_t e = tile / num_segs;
-    const uint32_t s = tile - e * num_segs;
-    const EntDesc ent = ents[e];
-    const SegDesc seg = segs[s];
-    if (!((seg.owner_mask >> ent.group) & 1ull)) continue;
-    const int64_t unit = seg.page_bytes / kpp[ent.group];
-    const int64_t off = unit * ent.first;
-    const int64_t len = unit * ent.valid;
-    char* dev = seg.base + ent.dev_block * seg.page_bytes + off;
-    char* host = host_base + ent.host_slot * host_stride + host_rank_offset +
-                 seg.host_offset + off;
+  for (uint32_t w = blockIdx.x; w < k.num_items; w += gridDim.x) {
+    const uint32_t tile = w / k.chunks_per_tile;
+    const uint32_t c = w - tile * k.chunks_per_tile;
+    const uint32_t e = tile / k.num_segs;
+    const uint32_t s = tile - e * k.num_segs;
+    const int32_t group = ents[e].group;
+    const int64_t page = segs[s].page_bytes;
+    if (!((segs[s].owner_mask >> group) & 1ull)) continue;
+    const int64_t unit = page / kpp[group];
+    const int64_t off = unit * ents[e].first;
+    const int64_t len = unit * ents[e].valid;
+    char* dev = segs[s].base + ents[e].dev_block * page + off;
+    char* host = k.host_base + ents[e].host_slot * k.host_stride + k.host_rank_offset +
+                 segs[s].host_offset + off;
     const char* src = TO_HOST ? dev : host;
     char* dst = TO_HOST ? host : dev;
     if (VEC) {
@@ -376,10 +391,53 @@ __global__ __launch_bounds__(WG) void swap_tiles_kernel(
           static_cast<uint32_t>((len - begin < kChunk) ? (len - begin) : kChunk);
       move_chunk16<WG, U, NT_STORE>(src + begin, dst + begin, nbytes);
     } else {
-      const Extent x = any_chunk<kChunk>(dst, len, c, chunks_per_tile - 1);
+      const Extent x = any_chunk<kChunk>(dst, len, c, k.chunks_per_tile - 1);
       if (x.nbytes) move_any<WG, U, NT_STORE>(src + x.begin, dst + x.begin, x.nbytes);
     }
   }
+}
+
+// `seen`: the guard's value as the descriptor's staging kernel found it (a
+// STAGED gather or scatter, over a full grid); `guard`: the guard itself (a
+// DIRECT swap, over a few persistent workgroups). Either may be null.
+template <int WG, int U, bool TO_HOST, bool VEC, bool NT_STORE>
+__global__ __launch_bounds__(WG) void swap_tiles_kernel(
+    const SegDesc* __restrict__ segs, const EntDesc* __restrict__ ents,
+    const int64_t* __restrict__ kpp, SwapWalk walk, const uint64_t* seen,
+    const uint64_t* guard) {
+  if (guard_set(seen) || guard_set_at_source(guard)) return;
+  swap_items<WG, U, TO_HOST, VEC, NT_STORE>(segs, ents, kpp, walk);
+}
+
+// A short DIRECT swap's whole descriptor in the kernel's own arguments, as
+// InlineCopy below: one launch. 72 segments and 45 entries.
+//
+// While the link is full, whatever the GPU fetches from host memory waits
+// behind the transfers (100-200 us a time), a launch's packet and a staged
+// descriptor among them, so a launch less counts double there.
+constexpr uint32_t kInlineSwapBytes = 3776;
+struct alignas(16) InlineSwap {
+  SwapWalk walk;
+  uint32_t kpp_offset, ent_offset;
+  uint32_t pad;
+  const uint64_t* guard;
+  unsigned char data[kInlineSwapBytes];
+};
+static_assert(offsetof(InlineSwap, data) % 16 == 0 && sizeof(InlineSwap) <= 3840,
+              "InlineSwap layout: 4 KiB of arguments, 256 bytes of them hidden ones");
+typedef __attribute__((address_space(4))) const char kernarg_char;
+
+template <bool TO_HOST, bool VEC, bool NT_STORE>
+__global__ __launch_bounds__(256) void swap_inline_kernel(InlineSwap a) {
+  typedef __attribute__((address_space(4))) const SegDesc kernarg_seg_desc;
+  typedef __attribute__((address_space(4))) const EntDesc kernarg_ent;
+  typedef __attribute__((address_space(4))) const int64_t kernarg_i64;
+  if (guard_set_at_source(a.guard)) return;
+  kernarg_char* data =
+      (kernarg_char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(InlineSwap, data);
+  swap_items<256, 2, TO_HOST, VEC, NT_STORE>((kernarg_seg_desc*)data,
+                                             (kernarg_ent*)(data + a.ent_offset),
+                                             (kernarg_i64*)(data + a.kpp_offset), a.walk);
 }
 
 // The order in which copy_blocks walks its work items, chosen on the host
@@ -471,7 +529,6 @@ struct alignas(16) InlineCopy {
 };
 static_assert(offsetof(InlineCopy, data) == 32 && sizeof(InlineCopy) <= 4096,
               "InlineCopy layout");
-typedef __attribute__((address_space(4))) const char kernarg_char;
 typedef __attribute__((address_space(4))) const CopySeg kernarg_seg;
 typedef __attribute__((address_space(4))) const PairDesc kernarg_pair;
 
@@ -1089,10 +1146,9 @@ struct SwapArgs {
   const SegDesc* segs;
   const EntDesc* ents;
   const int64_t* kpp;
-  uint32_t num_segs, num_items, cpt;
-  char* host_base;
-  int64_t host_stride, host_rank_offset;
-  const uint64_t* guard;
+  SwapWalk walk;
+  const uint64_t* seen;   // the staged guard value, or null
+  const uint64_t* guard;  // the guard itself, or null
 };
 
 template <int WG, int U, bool TO_HOST, bool VEC, bool NT>
@@ -1100,9 +1156,28 @@ hipError_t launch_swap_t(int64_t grid, hipStream_t st, const SwapArgs& a) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
   hipLaunchKernelGGL((swap_tiles_kernel<WG, U, TO_HOST, VEC, NT>),
                      dim3(static_cast<uint32_t>(grid)), dim3(WG), 0, st, a.segs, a.ents, a.kpp,
-                     a.num_segs, a.num_items, a.cpt, a.host_base, a.host_stride,
-                     a.host_rank_offset, a.guard);
+                     a.walk, a.seen, a.guard);
   return hipGetLastError();
+}
+
+template <bool TO_HOST, bool VEC, bool NT>
+hipError_t launch_inline_swap_t(int64_t grid, hipStream_t st, const InlineSwap& a) {
+  (void)hipGetLastError();  // clear a stale error: the check below is for this launch
+  hipLaunchKernelGGL((swap_inline_kernel<TO_HOST, VEC, NT>), dim3(static_cast<uint32_t>(grid)),
+                     dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_inline_swap(bool to_host, bool vec, bool nt, int64_t grid, hipStream_t st,
+                              const InlineSwap& a) {
+  if (to_host)  // never with non-temporal stores: the target is the host pool
+    return vec ? launch_inline_swap_t<true, true, false>(grid, st, a)
+               : launch_inline_swap_t<true, false, false>(grid, st, a);
+  if (nt)
+    return vec ? launch_inline_swap_t<false, true, true>(grid, st, a)
+               : launch_inline_swap_t<false, false, true>(grid, st, a);
+  return vec ? launch_inline_swap_t<false, true, false>(grid, st, a)
+             : launch_inline_swap_t<false, false, false>(grid, st, a);
 }
 
 template <int WG, int U>
@@ -1390,8 +1465,43 @@ struct Run {
   int64_t len;
 };
 
-// Enqueue one descriptor upload + kernel for entries [idx...] resolved to
+// The tables of a swap of entries order[lo, hi), at h: segments, then kernel
+// blocks per page, then entries resolved to the given host side.
+void pack_swap_desc(char* h, size_t kpp_off, size_t ent_off, const SwapLayout& L,
+                    const SwapList& E, const std::vector<int64_t>& order, size_t lo, size_t hi,
+                    bool is_swap_in, bool staged) {
+  SegDesc* hs = reinterpret_cast<SegDesc*>(h);
+  for (int32_t s = 0; s < L.num_segments; ++s)
+    hs[s] = SegDesc{static_cast<char*>(L.bases[s]), L.page_bytes[s], L.host_offsets[s],
+                    L.owner_masks[s]};
+  std::memcpy(h + kpp_off, L.kpp, sizeof(int64_t) * L.num_groups);
+  EntDesc* he = reinterpret_cast<EntDesc*>(h + ent_off);
+  for (size_t j = 0; j < hi - lo; ++j) {
+    const int64_t i = order[lo + j];
+    const int32_t g = E.group ? E.group[i] : 0;
+    EntDesc d;
+    d.dev_block = is_swap_in ? E.dst[i] : E.src[i];
+    const int64_t host_id = is_swap_in ? E.src[i] : E.dst[i];
+    d.host_slot = staged ? static_cast<int64_t>(j) : host_id;
+    d.group = g;
+    d.first = static_cast<int32_t>(E.first ? E.first[i] : 0);
+    d.valid = static_cast<int32_t>(E.valid ? E.valid[i] : L.kpp[g]);
+    d.pad = 0;
+    he[j] = d;
+  }
+}
+
+// Enqueue the descriptor and the kernel for entries order[lo, hi) resolved to
 // the given host side. Caller holds ctx->mu.
+//
+// A DIRECT swap's descriptor reaches the device inside the launch where it is
+// short, else by a runtime copy: those of a swap-out and a swap-in enqueued
+// together are both done (5.5 us each) before either fills the link. A
+// staging kernel read the second one from the host while the first swap had
+// the link, for 500-890 us (a model switch in a process with other swappers:
+// 12.4 ms, 11.9 so). A swap-out of one block of 72 x 32 KiB takes 68 us a
+// pass in one launch, 77 in two. STAGED kernels keep the staging kernel,
+// which reads the guard once for their full grids.
 int enqueue_swap_kernel(DeviceCtx* ctx, const SwapLayout& L, const SwapList& E,
                         const std::vector<int64_t>& order, size_t lo, size_t hi,
                         bool is_swap_in, bool staged, char* host_side, int64_t host_stride,
@@ -1399,61 +1509,60 @@ int enqueue_swap_kernel(DeviceCtx* ctx, const SwapLayout& L, const SwapList& E,
   const int32_t S = L.num_segments;
   const int64_t n = static_cast<int64_t>(hi - lo);
   if (n == 0) return 0;
-  const size_t seg_bytes = sizeof(SegDesc) * S;
-  const size_t kpp_off = (seg_bytes + 255) & ~size_t(255);
-  const size_t kpp_bytes = sizeof(int64_t) * L.num_groups;
-  const size_t ent_off = (kpp_off + kpp_bytes + 255) & ~size_t(255);
-  Desc desc;
-  int rc = desc_reserve(ctx->ring, ent_off + sizeof(EntDesc) * n, &desc);
-  if (rc) return rc;
-  char* h = ctx->ring.host + desc.off;
-  SegDesc* hs = reinterpret_cast<SegDesc*>(h);
-  int64_t max_page = 0;
-  for (int32_t s = 0; s < S; ++s) {
-    hs[s].base = static_cast<char*>(L.bases[s]);
-    hs[s].page_bytes = L.page_bytes[s];
-    hs[s].host_offset = L.host_offsets[s];
-    hs[s].owner_mask = L.owner_masks[s];
-    max_page = std::max(max_page, L.page_bytes[s]);
-  }
-  std::memcpy(h + kpp_off, L.kpp, kpp_bytes);
-  EntDesc* he = reinterpret_cast<EntDesc*>(h + ent_off);
-  for (int64_t j = 0; j < n; ++j) {
-    const int64_t i = order[lo + j];
-    const int32_t g = E.group ? E.group[i] : 0;
-    EntDesc d;
-    d.dev_block = is_swap_in ? E.dst[i] : E.src[i];
-    const int64_t host_id = is_swap_in ? E.src[i] : E.dst[i];
-    d.host_slot = staged ? j : host_id;
-    d.group = g;
-    d.first = static_cast<int32_t>(E.first ? E.first[i] : 0);
-    d.valid = static_cast<int32_t>(E.valid ? E.valid[i] : L.kpp[g]);
-    d.pad = 0;
-    he[j] = d;
-  }
-  char* dv = ctx->ring.dev + desc.off;
   const Tunables t = tunables();
+  int64_t max_page = 0;
+  for (int32_t s = 0; s < S; ++s) max_page = std::max(max_page, L.page_bytes[s]);
   const ShapeSel sh = swap_shape(t, vec, max_page);
   const int64_t cpt = (max_page + sh.chunk() - 1) / sh.chunk();
   const int64_t items = launch_items(n, S, cpt);
-  if (items < 0) {
-    ctx->ring.head = desc.off;  // nothing was enqueued; hand the region back
-    return too_many_items(n, S, cpt, "entries");
-  }
-  const uint64_t* guard = nullptr;
-  rc = desc_stage(ctx->ring, desc, E.guard, &guard, stream);
-  if (rc) return rc;
-  SwapArgs a{reinterpret_cast<const SegDesc*>(dv), reinterpret_cast<const EntDesc*>(dv + ent_off),
-             reinterpret_cast<const int64_t*>(dv + kpp_off), static_cast<uint32_t>(S),
-             static_cast<uint32_t>(items), static_cast<uint32_t>(cpt), host_side, host_stride,
-             host_rank_off, guard};
+  if (items < 0) return too_many_items(n, S, cpt, "entries");
+  const int64_t grid = launch_grid(wgs, items, sh.wg);
+  const SwapWalk walk{host_side, host_stride, host_rank_off, static_cast<uint32_t>(S),
+                      static_cast<uint32_t>(items), static_cast<uint32_t>(cpt)};
   // Non-temporal stores only where the destination is HBM: plain stores to
   // the host pool measured faster (no L2 residency to avoid there).
   const bool nt = t.nt_stores != 0 && !(!is_swap_in && !staged);
-  const hipError_t e =
-      launch_swap(sh, !is_swap_in, vec, nt, launch_grid(wgs, items, sh.wg), stream, a);
+  const size_t seg_bytes = sizeof(SegDesc) * S;
+  const size_t kpp_bytes = sizeof(int64_t) * L.num_groups;
+  const size_t ent_bytes = sizeof(EntDesc) * n;
+
+  const size_t short_ent_off = (seg_bytes + kpp_bytes + 15) & ~size_t(15);
+  if (!staged && sh.wg == 256 && sh.u == 2 && short_ent_off + ent_bytes <= kInlineSwapBytes) {
+    InlineSwap a;
+    a.walk = walk;
+    a.kpp_offset = static_cast<uint32_t>(seg_bytes);
+    a.ent_offset = static_cast<uint32_t>(short_ent_off);
+    a.pad = 0;
+    a.guard = E.guard;
+    pack_swap_desc(reinterpret_cast<char*>(a.data), seg_bytes, short_ent_off, L, E, order, lo, hi,
+                   is_swap_in, false);
+    const hipError_t e = launch_inline_swap(!is_swap_in, vec, nt, grid, stream, a);
+    return e == hipSuccess ? 0 : hip_fail(e, "swap_inline_kernel launch");
+  }
+
+  const size_t kpp_off = (seg_bytes + 255) & ~size_t(255);
+  const size_t ent_off = (kpp_off + kpp_bytes + 255) & ~size_t(255);
+  Desc desc;
+  int rc = desc_reserve(ctx->ring, ent_off + ent_bytes, &desc);
+  if (rc) return rc;
+  pack_swap_desc(ctx->ring.host + desc.off, kpp_off, ent_off, L, E, order, lo, hi, is_swap_in,
+                 staged);
+  char* dv = ctx->ring.dev + desc.off;
+  const uint64_t* seen = nullptr;
+  if (staged) {
+    rc = desc_stage(ctx->ring, desc, E.guard, &seen, stream);
+    if (rc) return rc;
+  } else {
+    AEGKV_HIP(hipMemcpyAsync(dv, ctx->ring.host + desc.off, desc.bytes, hipMemcpyHostToDevice,
+                             stream));
+  }
+  SwapArgs a{reinterpret_cast<const SegDesc*>(dv), reinterpret_cast<const EntDesc*>(dv + ent_off),
+             reinterpret_cast<const int64_t*>(dv + kpp_off), walk, seen,
+             staged ? nullptr : E.guard};
+  const hipError_t e = launch_swap(sh, !is_swap_in, vec, nt, grid, stream, a);
   if (e != hipSuccess) {
-    // the descriptor's staging is already enqueued: retire its region in order
+    // the descriptor's way to the device is already enqueued: retire its
+    // region in order
     (void)hipGetLastError();
     (void)ring_commit(ctx->ring, desc.off, desc.total(), stream);
     return hip_fail(e, "swap_tiles_kernel launch");
