@@ -217,44 +217,93 @@ struct Shape {
   static constexpr int64_t kChunk = int64_t(WG) * 16 * U;
 };
 
-template <bool NT_STORE>
-__device__ __forceinline__ void store16(gv4u* d, v4u x) {
-  if (NT_STORE)
-    __builtin_nontemporal_store(x, d);
-  else
-    *d = x;
+// Where the 16-byte words of one chunk go and how they are stored; `dst` and
+// `nbytes` are the same for the whole workgroup.
+//   kPlain:     targets in the host pool
+//   kStreaming: non-temporal, targets in HBM
+//   kThrough:   also at device scope, so that the L2 writes whole lines through
+//               as they come instead of keeping them for a later write-back.
+//               Only buffer stores can be told so.
+// Copies of random blocks, streaming -> through (TB/s, read plus written): 16
+// KiB pages 5.88 -> 5.99, 20 KiB 5.90 -> 5.98, 32 KiB 6.04 -> 6.12, 64 KiB 6.27
+// -> 6.42, 160 KiB 6.40 -> 6.57; plain stores 5.1-5.6. The scope bits of the
+// loads change nothing. Tiles that
+// do not begin and end on 128-byte lines write lines in parts, and lose by it
+// (16,388-byte pages 5.7 -> 5.2, 16,400 5.5 -> 5.4), as do shapes with several
+// loads per lane on few CUs (8 of 32 per XCD: 3.14 -> 3.04): these stay
+// streaming.
+enum StoreKind { kPlain, kStreaming, kThrough };
+constexpr int kBufferNt = 2, kBufferDeviceScope = 16;  // cache bits of a buffer store
+constexpr int kRawBufferWord3 = 0x00027000;            // untyped 32-bit data, no swizzle
+
+template <StoreKind K>
+struct Words {
+  gv4u* d;
+  __device__ __forceinline__ Words(char* dst, uint32_t, bool) : d((gv4u*)dst) {}
+  __device__ __forceinline__ void put(uint32_t i, v4u x) const {
+    if (K == kStreaming)
+      __builtin_nontemporal_store(x, d + i);
+    else
+      d[i] = x;
+  }
+};
+
+template <>
+struct Words<kThrough> {
+  __amdgpu_buffer_rsrc_t r;
+  bool lines;  // the tile is made of whole 128-byte lines
+  __device__ __forceinline__ Words(char* dst, uint32_t nbytes, bool whole_lines)
+      : r(__builtin_amdgcn_make_buffer_rsrc(dst, 0, static_cast<int>(nbytes), kRawBufferWord3)),
+        lines(whole_lines) {}
+  __device__ __forceinline__ void put(uint32_t i, v4u x) const {
+    const int at = static_cast<int>(i * 16u);
+    if (lines)
+      __builtin_amdgcn_raw_buffer_store_b128(x, r, at, 0, kBufferNt | kBufferDeviceScope);
+    else
+      __builtin_amdgcn_raw_buffer_store_b128(x, r, at, 0, kBufferNt);
+  }
+};
+
+__device__ __forceinline__ bool whole_lines(const char* tile, int64_t bytes) {
+  return ((reinterpret_cast<uintptr_t>(tile) | static_cast<uintptr_t>(bytes)) & 127u) == 0;
 }
+
+// The stores of a shape: through the L2 with one load per lane.
+template <int WG, int U, bool NT_STORE>
+using ShapeWords = Words<!NT_STORE ? kPlain : U == 1 && WG <= 256 ? kThrough : kStreaming>;
 
 // The guarded U loads of a tail chunk, all issued before the first store.
 // Recursion keeps every value in registers of its own: an array of U values
 // filled under conditions became one wide value that was copied whole at each
 // (252 VGPRs for U = 8, and with 1024 lanes scratch memory: 128 KiB tiles
 // copied at 1.3 TB/s).
-template <int WG, int U, bool NT_STORE>
-__device__ __forceinline__ void move_tail16(const gv4u* s, gv4u* d, uint32_t i, uint32_t n16) {
+template <int WG, int U, typename Out>
+__device__ __forceinline__ void move_tail16(const gv4u* s, const Out& d, uint32_t i,
+                                            uint32_t n16) {
   v4u x;
   if (i < n16) x = __builtin_nontemporal_load(s + i);
-  if constexpr (U > 1) move_tail16<WG, U - 1, NT_STORE>(s, d, i + WG, n16);
-  if (i < n16) store16<NT_STORE>(d + i, x);
+  if constexpr (U > 1) move_tail16<WG, U - 1>(s, d, i + WG, n16);
+  if (i < n16) d.put(i, x);
 }
 
 // Move nbytes (multiple of 16, at most one chunk) with 16 B per lane. A full
 // chunk issues all U loads back to back before the first store; only a tail
 // chunk pays for per-load guards.
 template <int WG, int U, bool NT_STORE>
-__device__ __forceinline__ void move_chunk16(const char* src, char* dst, uint32_t nbytes) {
+__device__ __forceinline__ void move_chunk16(const char* src, char* dst, uint32_t nbytes,
+                                             bool lines = false) {
   const gv4u* s = (const gv4u*)src;  // generic -> global address space
-  gv4u* d = (gv4u*)dst;
+  const ShapeWords<WG, U, NT_STORE> d(dst, nbytes, lines);
   const uint32_t tid = threadIdx.x;
   if (nbytes != static_cast<uint32_t>(Shape<WG, U>::kChunk)) {
-    move_tail16<WG, U, NT_STORE>(s, d, tid, nbytes >> 4);
+    move_tail16<WG, U>(s, d, tid, nbytes >> 4);
     return;
   }
   v4u r[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) r[u] = __builtin_nontemporal_load(s + tid + u * WG);
 #pragma unroll
-  for (int u = 0; u < U; ++u) store16<NT_STORE>(d + tid + u * WG, r[u]);
+  for (int u = 0; u < U; ++u) d.put(tid + u * WG, r[u]);
 }
 
 // A move guard is a word a stream's fence waits set when they give up or
@@ -326,7 +375,7 @@ __device__ __forceinline__ void move_any(const char* src, char* dst, uint32_t nb
   char b = 0;
   if (edge) b = ((const gchar*)src)[at];
   const gchar* s = (const gchar*)src + head;
-  gv4u* d = (gv4u*)(dst + head);
+  const Words<NT_STORE ? kStreaming : kPlain> d(dst + head, n16 * 16u, false);
   uint32_t i = tid;
   for (; i + (U - 1) * WG < n16; i += U * WG) {
     v4u r[U];
@@ -334,10 +383,10 @@ __device__ __forceinline__ void move_any(const char* src, char* dst, uint32_t nb
     for (int u = 0; u < U; ++u)
       r[u] = __builtin_nontemporal_load((const gv4u_any*)(s + (i + u * WG) * 16u));
 #pragma unroll
-    for (int u = 0; u < U; ++u) store16<NT_STORE>(d + i + u * WG, r[u]);
+    for (int u = 0; u < U; ++u) d.put(i + u * WG, r[u]);
   }
   for (; i < n16; i += WG)
-    store16<NT_STORE>(d + i, __builtin_nontemporal_load((const gv4u_any*)(s + i * 16u)));
+    d.put(i, __builtin_nontemporal_load((const gv4u_any*)(s + i * 16u)));
   if (edge) ((gchar*)dst)[at] = b;
 }
 
@@ -452,6 +501,7 @@ __global__ __launch_bounds__(256) void swap_inline_kernel(InlineSwap a) {
 // written, 4 KiB items): 160 KiB tiles 5.24 -> 6.45, 64 KiB 5.87 -> 6.19,
 // 32 KiB 5.44 -> 5.88, 20 KiB 5.36 -> 6.01, 16 KiB 5.43 -> 5.99, 4 KiB
 // 5.60 -> 6.15. Segment order alone gives 0-6 % of that, runs alone 2-4 %.
+// (Measured with streaming stores; Words has what storing through adds.)
 struct CopyWalk {
   uint32_t num_pairs;
   uint32_t num_items;
@@ -493,7 +543,7 @@ __device__ __forceinline__ void copy_items(Segs segs, Pairs pairs, const CopyWal
       if (begin >= page) continue;
       const uint32_t nbytes =
           static_cast<uint32_t>((page - begin < kChunk) ? (page - begin) : kChunk);
-      move_chunk16<WG, U, NT_STORE>(src + begin, dst + begin, nbytes);
+      move_chunk16<WG, U, NT_STORE>(src + begin, dst + begin, nbytes, whole_lines(dst, page));
     } else {
       const Extent x = any_chunk<kChunk>(dst, page, it.chunk, walk.chunks_per_tile - 1);
       if (x.nbytes) move_any<WG, U, NT_STORE>(src + x.begin, dst + x.begin, x.nbytes);
@@ -580,16 +630,13 @@ __global__ __launch_bounds__(WG) void copy_probe_kernel(const CopySeg* __restric
 #pragma unroll
       for (int u = 0; u < U; ++u) acc ^= r[u];
     } else {
-      gv4u* dst = (gv4u*)(seg.dst + pr.dst * seg.page_bytes + begin);
+      char* tile = seg.dst + pr.dst * seg.page_bytes;
+      const ShapeWords<WG, U, NT_STORE> dst(tile + begin, n16 * 16u,
+                                            whole_lines(tile, seg.page_bytes));
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const uint32_t i = tid + u * WG;
-        if (i < n16) {
-          if (NT_STORE)
-            __builtin_nontemporal_store(pattern, dst + i);
-          else
-            dst[i] = pattern;
-        }
+        if (i < n16) dst.put(i, pattern);
       }
     }
   }
@@ -719,8 +766,8 @@ ShapeSel auto_shape(int64_t page) {
 // wave) where pages are no multiple of 4 KiB and 4 KiB items would leave
 // lanes idle in the last one. In the order of copy_item, few bytes per item
 // keep what the chip writes at any moment close together: 160 KiB tiles run
-// at 6.45 TB/s with 4 KiB items, 6.18 with 8 or 16 KiB, 6.03 with one item
-// a tile; 12.5 KiB tiles at 5.69 with 4 KiB items and 6.02 with 1 KiB, 1 KiB
+// at 6.45 TB/s (streaming stores) with 4 KiB items, 6.18 with 8 or 16 KiB,
+// 6.03 with one item a tile; 12.5 KiB tiles at 5.69 with 4 KiB items and 6.02 with 1 KiB, 1 KiB
 // tiles at 3.84 and 6.19. On multiples of 4 KiB the two are within 1 %.
 //
 // One load per lane keeps 32 KiB in flight on a CU, which fills the chip's

@@ -404,6 +404,38 @@ def test_copy_on_a_masked_stream_vs_expectation(gpu, page):
         masked.close()
 
 
+@pytest.mark.parametrize("shift", [0, 16, 64, 128])
+@pytest.mark.parametrize("page", [16, 112, 128, 144, 1024, 1152, 4096, 4224, 4208, 16400, 20480])
+def test_copies_of_whole_lines_and_others(gpu, page, shift):
+    """Tiles made of whole 128-byte lines are stored another way than others:
+    pages and starts on and off lines, segments of both kinds in one call,
+    tails of one line, and nothing outside the target pages touched."""
+    _say("whole lines", page, shift)
+    g = torch.Generator(device=gpu).manual_seed(page + shift)
+    rng = np.random.default_rng(page + shift)
+    n, m = 30, 13
+    ids = rng.permutation(n)
+    src, dst = ids[:m], ids[m:2 * m]
+    s, d = torch.from_numpy(src.copy()).to(gpu), torch.from_numpy(dst.copy()).to(gpu)
+    for long in (False, True):   # the descriptor in the launch, and staged
+        k = 1 if not long else 112
+        wholes = [torch.randint(0, 256, (256 + n * page + 256,), dtype=torch.uint8, device=gpu,
+                                generator=g) for _ in range(2 * k)]
+        starts = [128 + (shift if i % 2 else 0) for i in range(2 * k)]
+        segs = [w[b:b + n * page].view(n, page) for w, b in zip(wholes, starts)]
+        want = [w.clone() for w in wholes]
+        for w, b in zip(want, starts):
+            rows = w[b:b + n * page].view(n, page)
+            rows[d] = rows[s]
+        for entry in (ops.copy_blocks, ops.copy_blocks_noalloc):
+            kept = [w.clone() for w in wholes]
+            entry(segs, src, dst)
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(wholes, want)), (entry.__name__, long)
+            for w, k0 in zip(wholes, kept):
+                w.copy_(k0)
+
+
 class _Sub(torch.Tensor):
     pass
 
