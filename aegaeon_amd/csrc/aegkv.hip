@@ -307,10 +307,12 @@ __device__ __forceinline__ void move_chunk16(const char* src, char* dst, uint32_
 }
 
 // A move guard is a word a stream's fence waits set when they give up or
-// see a failed source (aegkv_fence_wait). The descriptor's staging kernel
-// reads it once per launch, at system scope (it may live in pinned host
-// memory), into a device word behind the descriptor; the moving kernels test
-// that word and move nothing when it is set.
+// see a failed source (aegkv_fence_wait). Kernels over full grids
+// (migrations, STAGED gathers and scatters) move nothing when the word that
+// their descriptor's staging kernel left is set: that kernel reads the guard
+// once per launch, at system scope (it may live in pinned host memory), into
+// a device word behind the descriptor. DIRECT swaps, over a few persistent
+// workgroups, read the guard themselves (guard_set_at_source).
 //
 // Read by every wave of the moving kernel instead, a guard in pinned host
 // memory costs 83-88 ns per wave, one after another whatever the grid: a
