@@ -145,4 +145,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostargs", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__hostargs() { return PyModule_Create(&module); }
+// torch_version: the torch whose tensor layout this was compiled against.
+PyMODINIT_FUNC PyInit__hostargs() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", AEGKV_TORCH_VERSION) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -485,6 +485,37 @@ def test_segment_table_reads_what_the_general_path_reads(gpu):
         assert all(torch.equal(x, y) for x, y in zip(got, want[1:]))
 
 
+def test_moves_without_the_native_readers(gpu, monkeypatch):
+    """Where _hostargs.so cannot be used, lists of integers and plain device
+    tensors take the general path to the same bytes."""
+    from aegaeon_amd import _lib
+
+    g = torch.Generator(device=gpu).manual_seed(5)
+    a = [torch.randint(0, 256, (9, 64 * (s + 1)), dtype=torch.uint8, device=gpu, generator=g)
+         for s in range(3)]
+    pages = [64, 128, 192]
+    pool = ops.PinnedHostPool(9 * sum(pages))
+
+    def moves():
+        segs = [t.clone() for t in a]
+        pool.tensor.zero_()
+        lay = ops.SegmentLayout(segs, pages, [0, 64, 192], [1, 1, 1], 9, [1], pool.tensor,
+                                sum(pages), 0)
+        ops.copy_blocks(segs, [0, 1], [2, 3])
+        ops.copy_blocks_noalloc(segs, [4], [5])
+        ops.migrate_blocks(a, segs, [8], [6])
+        lay.swap([2, 5], [1, 7], [0, 0], [0, 0], [1, 1], False)
+        lay.swap([7], [4], [0], [0], [1], True)
+        torch.cuda.synchronize()
+        return segs + [pool.tensor.clone()]
+
+    want = moves()
+    assert int((want[-1] != 0).sum()) > 300 and not torch.equal(want[0], a[0])
+    monkeypatch.setattr(_lib, "_hostargs", _lib._GeneralPath)
+    assert all(torch.equal(x, y) for x, y in zip(moves(), want))
+    torch.cuda.synchronize()
+
+
 def _shifted(nbytes, shift, device, g):
     """Random device bytes starting `shift` bytes behind a 16-byte boundary,
     with 64 bytes around them that no move may touch: (all, the view)."""

@@ -929,3 +929,78 @@ def test_segment_table_leaves_host_tensors_to_the_general_path(aegkv_lib):
         assert table(segs, None) is None
     with pytest.raises(ValueError, match="device"):
         ops.copy_blocks([torch.zeros(4, 8)], [0], [1])
+
+
+@pytest.fixture
+def no_hostargs(monkeypatch):
+    """A package whose _hostargs.so is missing."""
+    import sys
+
+    import aegaeon_amd
+    from aegaeon_amd import _lib
+
+    monkeypatch.setattr(_lib, "_hostargs", None)
+    monkeypatch.delattr(aegaeon_amd, "_hostargs", raising=False)
+    monkeypatch.setitem(sys.modules, "aegaeon_amd._hostargs", None)
+    return _lib
+
+
+def test_arguments_are_read_without_the_native_readers(aegkv_lib, no_hostargs):
+    """The native readers only save time: without them one warning is given
+    and every reader leaves its argument to the general path."""
+    import warnings
+
+    from aegaeon_amd import ops
+
+    with pytest.warns(RuntimeWarning, match="_hostargs.so is not used"):
+        arg, n = ops._id_arg([3, 1, 2])
+    assert [arg[i] for i in range(n)] == [3, 1, 2]
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")   # told once
+        arg, n = ops._group_arg((0, 5))
+        assert [arg[i] for i in range(n)] == [0, 5]
+        with pytest.raises(ValueError, match="device"):
+            ops.copy_blocks([torch.zeros(4, 8)], [0], [1])
+        with pytest.raises(ValueError, match="device"):
+            ops.migrate_blocks([torch.zeros(4, 8)], [torch.zeros(4, 8)], [0], [1])
+
+
+def test_native_readers_of_another_torch_are_not_used(aegkv_lib, monkeypatch):
+    """They read tensors through torch's own layout, which is one version's."""
+    from aegaeon_amd import _lib, ops
+
+    assert _lib.hostargs().torch_version == torch.__version__
+    monkeypatch.setattr(_lib, "_hostargs", None)
+    monkeypatch.setattr(torch, "__version__", "0.0")
+    with pytest.warns(RuntimeWarning, match="built for torch"):
+        arg, n = ops._id_arg([7])
+    assert n == 1 and arg[0] == 7
+
+
+@pytest.mark.parametrize("fault", [OSError("g++: not found"), 1])
+def test_the_library_is_built_without_the_native_readers(tmp_path, monkeypatch, fault):
+    """g++ or torch's headers missing: libaegkv.so is there all the same, and
+    no _hostargs.so of an earlier build stays beside it."""
+    import subprocess
+    from pathlib import Path
+
+    from aegaeon_amd import build as lib_build
+
+    monkeypatch.setattr(lib_build, "LIB_PATH", tmp_path / "libaegkv.so")
+    monkeypatch.setattr(lib_build, "HOSTARGS_PATH", tmp_path / "_hostargs.so")
+    monkeypatch.setattr(lib_build, "hipcc", lambda: "hipcc")
+    (tmp_path / "_hostargs.so").write_text("an earlier build's")
+
+    def run(cmd, **kw):
+        if cmd[0] == "hipcc":
+            Path(cmd[cmd.index("-o") + 1]).write_text("built")
+            return subprocess.CompletedProcess(cmd, 0, "", "")
+        if isinstance(fault, OSError):
+            raise fault
+        return subprocess.CompletedProcess(cmd, fault, "", "no torch headers")
+
+    monkeypatch.setattr(lib_build.subprocess, "run", run)
+    with pytest.warns(RuntimeWarning, match="was not built"):
+        assert lib_build.build() == tmp_path / "libaegkv.so"
+    assert (tmp_path / "libaegkv.so").read_text() == "built"
+    assert not (tmp_path / "_hostargs.so").exists()
