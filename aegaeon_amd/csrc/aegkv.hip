@@ -27,6 +27,7 @@
 
 #include <hip/hip_runtime.h>
 #include "aegkv.h"
+#include "copy_walk.h"
 #include "errors.h"
 
 #include <algorithm>
@@ -338,26 +339,6 @@ __global__ __launch_bounds__(kStageLanes) void desc_stage_kernel(const v4u* __re
     *seen = __hip_atomic_load(guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Tiles whose addresses or lengths are no multiples of 16 (a cache whose
-// pages end in a scale, a pool that starts anywhere) are cut into chunks
-// where their *target* crosses 16-byte boundaries: only the first chunk of a
-// tile starts and only its last one ends inside a 16-byte word.
-struct Extent {
-  int64_t begin;
-  uint32_t nbytes;
-};
-
-// Chunk `c` of a `len`-byte tile; the chunk numbered `last` takes the rest.
-template <int64_t kChunk>
-__device__ __forceinline__ Extent any_chunk(const char* dst_tile, int64_t len, uint32_t c,
-                                            uint32_t last) {
-  const int64_t head = static_cast<int64_t>(-reinterpret_cast<uintptr_t>(dst_tile) & 15u);
-  const int64_t begin = c ? head + static_cast<int64_t>(c) * kChunk : 0;
-  const int64_t next = head + (static_cast<int64_t>(c) + 1) * kChunk;
-  const int64_t end = (c == last || next > len) ? len : next;
-  return {begin, begin < end ? static_cast<uint32_t>(end - begin) : 0u};
-}
-
 // Move nbytes from any address to any other: 16 B per lane, loads at the
 // source's own alignment (the hardware takes any) and stores on the target's
 // 16-byte words, with single bytes at both ends. 16,388-byte pages, one byte
@@ -491,48 +472,22 @@ __global__ __launch_bounds__(256) void swap_inline_kernel(InlineSwap a) {
                                              (kernarg_i64*)(data + a.kpp_offset), a.walk);
 }
 
-// The order in which copy_blocks walks its work items, chosen on the host
-// (copy_walk): segment by segment, the pairs of one segment in the order of
-// the descriptor, the chunks of one tile in address order. Workgroups are
-// handed to the 8 XCDs in turn, so items [0, remap_end) are renumbered to
-// give every XCD whole runs of 2^run_shift consecutive items: with pairs in
-// target order each XCD then writes one stretch of one segment at a time.
-//
-// HBM bounds the copy, and this order is what it answers best. Random halves
-// of a cache, against pairs-first items over the whole chip (TB/s, read plus
-// written, 4 KiB items): 160 KiB tiles 5.24 -> 6.45, 64 KiB 5.87 -> 6.19,
-// 32 KiB 5.44 -> 5.88, 20 KiB 5.36 -> 6.01, 16 KiB 5.43 -> 5.99, 4 KiB
-// 5.60 -> 6.15. Segment order alone gives 0-6 % of that, runs alone 2-4 %.
-// (Measured with streaming stores; Words has what storing through adds.)
-struct CopyWalk {
-  uint32_t num_pairs;
-  uint32_t num_items;
-  uint32_t chunks_per_tile;
-  uint32_t remap_end;
-  uint32_t run_shift;
-};
-
-struct CopyItem {
-  uint32_t pair, segment, chunk;
-};
-
-__device__ __forceinline__ CopyItem copy_item(const CopyWalk& k, uint32_t w) {
-  if (w < k.remap_end) {
-    const uint32_t r = w & ((8u << k.run_shift) - 1u);
-    w = w - r + ((r & 7u) << k.run_shift) + (r >> 3);
-  }
-  const uint32_t tile = w / k.chunks_per_tile;
-  const uint32_t s = tile / k.num_pairs;
-  return {tile - s * k.num_pairs, s, w - tile * k.chunks_per_tile};
+// The classes of a walk where the launch put them: the kernel's first
+// argument. Indexed as a parameter they would be copied to scratch memory.
+typedef __attribute__((address_space(4))) const CopyClass kernarg_class;
+__device__ __forceinline__ kernarg_class* first_argument() {
+  return (kernarg_class*)__builtin_amdgcn_kernarg_segment_ptr();
 }
 
 // copy_blocks: one item is one chunk of one (segment, pair) tile. The host
 // keeps num_items + gridDim.x below 2^32 (launch_items).
-template <int WG, int U, bool VEC, bool NT_STORE, typename Segs, typename Pairs>
-__device__ __forceinline__ void copy_items(Segs segs, Pairs pairs, const CopyWalk& walk) {
+template <int WG, int U, bool VEC, bool NT_STORE, typename Segs, typename Pairs,
+          typename Classes>
+__device__ __forceinline__ void copy_items(Segs segs, Pairs pairs, const CopyWalk& walk,
+                                           Classes classes, uint32_t num_classes) {
   constexpr int64_t kChunk = Shape<WG, U>::kChunk;
   for (uint32_t w = blockIdx.x; w < walk.num_items; w += gridDim.x) {
-    const CopyItem it = copy_item(walk, w);
+    const CopyItem it = copy_item(walk, classes, num_classes, w);
     const int64_t src_block = pairs[it.pair].src, dst_block = pairs[it.pair].dst;
     const int64_t page = segs[it.segment].page_bytes;
     const char* src = segs[it.segment].src + src_block * page;
@@ -547,23 +502,24 @@ __device__ __forceinline__ void copy_items(Segs segs, Pairs pairs, const CopyWal
           static_cast<uint32_t>((page - begin < kChunk) ? (page - begin) : kChunk);
       move_chunk16<WG, U, NT_STORE>(src + begin, dst + begin, nbytes, whole_lines(dst, page));
     } else {
-      const Extent x = any_chunk<kChunk>(dst, page, it.chunk, walk.chunks_per_tile - 1);
+      const Extent x = any_chunk<kChunk>(dst, page, it.chunk, it.last);
       if (x.nbytes) move_any<WG, U, NT_STORE>(src + x.begin, dst + x.begin, x.nbytes);
     }
   }
 }
 
 template <int WG, int U, bool VEC, bool NT_STORE>
-__global__ __launch_bounds__(WG) void copy_blocks_kernel(const CopySeg* __restrict__ segs,
+__global__ __launch_bounds__(WG) void copy_blocks_kernel(CopyClasses, uint32_t num_classes,
+                                                         const CopySeg* __restrict__ segs,
                                                          const PairDesc* __restrict__ pairs,
                                                          CopyWalk walk,
                                                          const uint64_t* __restrict__ guard) {
   if (guard_set(guard)) return;
-  copy_items<WG, U, VEC, NT_STORE>(segs, pairs, walk);
+  copy_items<WG, U, VEC, NT_STORE>(segs, pairs, walk, first_argument(), num_classes);
 }
 
-// A short copy's whole descriptor (segment table, then pair table) in the
-// kernel's own arguments, which the runtime copies when the launch is
+// A short copy's whole descriptor (segment table, classes of the walk behind
+// the first, pair table) in the kernel's own arguments, which the runtime copies when the launch is
 // enqueued (a graph that captures it keeps its own copy) and every workgroup
 // reads through the scalar cache: the call is one launch, with no upload in
 // front of it, no ring region and no event behind it.
@@ -575,8 +531,8 @@ __global__ __launch_bounds__(WG) void copy_blocks_kernel(const CopySeg* __restri
 constexpr uint32_t kInlineBytes = 3808;
 struct alignas(16) InlineCopy {
   CopyWalk walk;
-  uint32_t pair_offset;  // bytes of the segment table
-  uint32_t pad[2];
+  uint32_t pair_offset;  // bytes of the segment table and the classes
+  uint32_t num_classes;
   unsigned char data[kInlineBytes];
 };
 static_assert(offsetof(InlineCopy, data) == 32 && sizeof(InlineCopy) <= 4096,
@@ -590,8 +546,9 @@ __global__ __launch_bounds__(WG) void copy_blocks_inline_kernel(InlineCopy a) {
   // only argument and starts its argument segment
   kernarg_char* data =
       (kernarg_char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(InlineCopy, data);
-  copy_items<WG, 1, VEC, NT_STORE>((kernarg_seg*)data, (kernarg_pair*)(data + a.pair_offset),
-                                   a.walk);
+  kernarg_char* pairs = data + a.pair_offset;
+  copy_items<WG, 1, VEC, NT_STORE>((kernarg_seg*)data, (kernarg_pair*)pairs, a.walk,
+                                   (kernarg_class*)pairs - a.num_classes, a.num_classes);
 }
 
 // Measurement twins of copy_blocks_kernel (aegkv_copy_probe): the same
@@ -605,7 +562,8 @@ constexpr int PROBE_READ = 1;
 constexpr int PROBE_WRITE = 2;
 
 template <int WG, int U, int KIND, bool NT_STORE>
-__global__ __launch_bounds__(WG) void copy_probe_kernel(const CopySeg* __restrict__ segs,
+__global__ __launch_bounds__(WG) void copy_probe_kernel(CopyClasses, uint32_t num_classes,
+                                                        const CopySeg* __restrict__ segs,
                                                         const PairDesc* __restrict__ pairs,
                                                         CopyWalk walk, uint32_t* sink,
                                                         uint32_t magic) {
@@ -614,7 +572,7 @@ __global__ __launch_bounds__(WG) void copy_probe_kernel(const CopySeg* __restric
   v4u acc = {0u, 0u, 0u, 0u};
   const v4u pattern = {tid, blockIdx.x, 0x5a5a5a5au, magic};
   for (uint32_t w = blockIdx.x; w < walk.num_items; w += gridDim.x) {
-    const CopyItem it = copy_item(walk, w);
+    const CopyItem it = copy_item(walk, first_argument(), num_classes, w);
     const PairDesc pr = pairs[it.pair];
     const CopySeg seg = segs[it.segment];
     const int64_t begin = static_cast<int64_t>(it.chunk) * kChunk;
@@ -1167,23 +1125,6 @@ int64_t launch_grid(int64_t limit, int64_t items, int lanes) {
   return std::max<int64_t>(1, std::min<int64_t>(g, cap));
 }
 
-// Work items one launch may hold. The kernels walk items with a 32-bit
-// grid-stride loop (w += gridDim.x) and launch_grid caps a grid at
-// (2^32 - 1) / 256 workgroups, so with at most this many items,
-// w + gridDim.x stays below 2^32 and the loop never wraps.
-constexpr int64_t kMaxLaunchItems =
-    static_cast<int64_t>(UINT32_MAX) - static_cast<int64_t>(UINT32_MAX) / 256;
-
-// a * b * c work items, or -1 when that exceeds kMaxLaunchItems (or overflows).
-int64_t launch_items(int64_t a, int64_t b, int64_t c) {
-  if (a < 0 || b < 0 || c < 0) return -1;
-  if (a == 0 || b == 0 || c == 0) return 0;
-  if (a > kMaxLaunchItems / b) return -1;
-  const int64_t ab = a * b;
-  if (ab > kMaxLaunchItems / c) return -1;
-  return ab * c;
-}
-
 int too_many_items(int64_t a, int64_t b, int64_t c, const char* what) {
   return fail(AEGKV_EINVAL, "%lld %s x %lld segments x %lld chunks exceed the %lld work items "
               "of one launch; split the call", static_cast<long long>(a), what,
@@ -1261,27 +1202,27 @@ hipError_t launch_swap(ShapeSel sh, bool to_host, bool vec, bool nt, int64_t gri
 // caps how many workgroups share a CU.
 template <int WG, int U, bool VEC, bool NT>
 hipError_t launch_copy_t(int64_t grid, unsigned lds, hipStream_t st, const CopySeg* s,
-                         const PairDesc* p, const CopyWalk& walk, const uint64_t* guard) {
+                         const PairDesc* p, const CopyLayout& l, const uint64_t* guard) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
   hipLaunchKernelGGL((copy_blocks_kernel<WG, U, VEC, NT>), dim3(static_cast<uint32_t>(grid)),
-                     dim3(WG), lds, st, s, p, walk, guard);
+                     dim3(WG), lds, st, l.classes, l.num_classes, s, p, l.walk, guard);
   return hipGetLastError();
 }
 
 hipError_t launch_copy(ShapeSel sh, bool vec, bool nt, int64_t grid, unsigned lds,
-                       hipStream_t st, const CopySeg* s, const PairDesc* p, const CopyWalk& walk,
+                       hipStream_t st, const CopySeg* s, const PairDesc* p, const CopyLayout& l,
                        const uint64_t* guard) {
   if (!vec) {
     if (sh.wg == 64)
-      return nt ? launch_copy_t<64, 1, false, true>(grid, 0, st, s, p, walk, guard)
-                : launch_copy_t<64, 1, false, false>(grid, 0, st, s, p, walk, guard);
-    return nt ? launch_copy_t<256, 1, false, true>(grid, 0, st, s, p, walk, guard)
-              : launch_copy_t<256, 1, false, false>(grid, 0, st, s, p, walk, guard);
+      return nt ? launch_copy_t<64, 1, false, true>(grid, 0, st, s, p, l, guard)
+                : launch_copy_t<64, 1, false, false>(grid, 0, st, s, p, l, guard);
+    return nt ? launch_copy_t<256, 1, false, true>(grid, 0, st, s, p, l, guard)
+              : launch_copy_t<256, 1, false, false>(grid, 0, st, s, p, l, guard);
   }
 #define AEGKV_CP(W, UU)                                                               \
   if (sh.wg == W && sh.u == UU)                                                       \
-    return nt ? launch_copy_t<W, UU, true, true>(grid, lds, st, s, p, walk, guard)    \
-              : launch_copy_t<W, UU, true, false>(grid, lds, st, s, p, walk, guard);
+    return nt ? launch_copy_t<W, UU, true, true>(grid, lds, st, s, p, l, guard)       \
+              : launch_copy_t<W, UU, true, false>(grid, lds, st, s, p, l, guard);
   AEGKV_CP(64, 1) AEGKV_CP(256, 1) AEGKV_CP(256, 2) AEGKV_CP(256, 4) AEGKV_CP(256, 8)
   AEGKV_CP(1024, 1) AEGKV_CP(1024, 2) AEGKV_CP(1024, 3) AEGKV_CP(1024, 4)
   AEGKV_CP(1024, 5) AEGKV_CP(1024, 6) AEGKV_CP(1024, 8) AEGKV_CP(1024, 10)
@@ -1311,24 +1252,24 @@ hipError_t launch_inline(int lanes, bool vec, bool nt, int64_t grid, hipStream_t
 
 template <int WG, int U, int KIND, bool NT>
 hipError_t launch_probe_t(int64_t grid, unsigned lds, hipStream_t st, const CopySeg* s,
-                          const PairDesc* p, const CopyWalk& walk, uint32_t* sink,
+                          const PairDesc* p, const CopyLayout& l, uint32_t* sink,
                           uint32_t magic) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
   hipLaunchKernelGGL((copy_probe_kernel<WG, U, KIND, NT>), dim3(static_cast<uint32_t>(grid)),
-                     dim3(WG), lds, st, s, p, walk, sink, magic);
+                     dim3(WG), lds, st, l.classes, l.num_classes, s, p, l.walk, sink, magic);
   return hipGetLastError();
 }
 
 hipError_t launch_probe(ShapeSel sh, int kind, bool nt, int64_t grid, unsigned lds,
                         hipStream_t st, const CopySeg* s, const PairDesc* p,
-                        const CopyWalk& walk, uint32_t* sink, uint32_t magic) {
+                        const CopyLayout& l, uint32_t* sink, uint32_t magic) {
 #define AEGKV_PR(W, UU)                                                                        \
   if (sh.wg == W && sh.u == UU) {                                                              \
     if (kind == PROBE_READ)                                                                    \
-      return launch_probe_t<W, UU, PROBE_READ, false>(grid, lds, st, s, p, walk, sink, magic); \
-    return nt ? launch_probe_t<W, UU, PROBE_WRITE, true>(grid, lds, st, s, p, walk, sink,      \
+      return launch_probe_t<W, UU, PROBE_READ, false>(grid, lds, st, s, p, l, sink, magic); \
+    return nt ? launch_probe_t<W, UU, PROBE_WRITE, true>(grid, lds, st, s, p, l, sink,      \
                                                          magic)                                \
-              : launch_probe_t<W, UU, PROBE_WRITE, false>(grid, lds, st, s, p, walk, sink,     \
+              : launch_probe_t<W, UU, PROBE_WRITE, false>(grid, lds, st, s, p, l, sink,     \
                                                           magic);                              \
   }
   AEGKV_PR(64, 1) AEGKV_PR(256, 1) AEGKV_PR(256, 2) AEGKV_PR(256, 4) AEGKV_PR(256, 8)
@@ -2103,41 +2044,26 @@ int copy_check_device(int32_t num_segments, void* const* src_bases, void* const*
 struct CopyPlan {
   ShapeSel sh;
   bool vec;
-  int64_t items;  // work items (segment x pair x chunk)
-  CopyWalk walk;
+  CopyLayout lay;
 };
 
-// The walk of `items` items (see CopyWalk). Runs hold about 32 tiles: from 8
-// to 512 the rate moves by 2 % (least at 8 and 512 on 4-20 KiB tiles).
-CopyWalk copy_walk(int64_t num_pairs, int64_t cpt, int64_t items) {
-  uint32_t shift = 5;
-  while (shift < 20 && (int64_t(1) << shift) < 32 * cpt) ++shift;
-  const int64_t span = int64_t(8) << shift;
-  return CopyWalk{static_cast<uint32_t>(num_pairs), static_cast<uint32_t>(items),
-                  static_cast<uint32_t>(cpt), static_cast<uint32_t>(items / span * span), shift};
-}
-
-int copy_plan(const Tunables& t, bool vec, int64_t max_page, bool all_cus, int32_t num_segments,
-              int64_t num_pairs, CopyPlan* out) {
+int copy_plan(const Tunables& t, bool vec, const int64_t* page_bytes, int64_t max_page,
+              bool all_cus, int32_t num_segments, int64_t num_pairs, CopyPlan* out) {
+  out->vec = vec;
+  auto lay = [&](ShapeSel sh) {
+    out->sh = sh;
+    return lay_walk(page_bytes, num_segments, num_pairs, sh.chunk(), vec, &out->lay);
+  };
   ShapeSel sh = copy_shape(max_page, all_cus);
   if (t.copy_unroll > 0)
     sh = ShapeSel{t.copy_lanes == 256 ? 256 : 1024, static_cast<int>(t.copy_unroll)};
-  auto chunks = [&] { return (max_page + sh.chunk() - 1) / sh.chunk(); };
-  // unaligned tiles: the last chunk takes up to half a chunk more, so that
-  // a few bytes over do not cost a wave of their own
-  auto any_chunks = [&] { return std::max<int64_t>(1, (max_page + sh.chunk() / 2) / sh.chunk()); };
-  if (!vec) sh = ShapeSel{64, 1};
-  int64_t cpt = vec ? chunks() : any_chunks();
-  int64_t items = launch_items(num_pairs, num_segments, cpt);
-  if (items < 0 && (!vec || t.copy_unroll == 0)) {
+  if (lay(vec ? sh : ShapeSel{64, 1})) return 0;
+  if (!vec || t.copy_unroll == 0) {
     // more small items than one launch holds
-    sh = vec ? auto_shape(max_page) : ShapeSel{256, 1};
-    cpt = vec ? chunks() : any_chunks();
-    items = launch_items(num_pairs, num_segments, cpt);
+    if (lay(vec ? auto_shape(max_page) : ShapeSel{256, 1})) return 0;
   }
-  if (items < 0) return too_many_items(num_pairs, num_segments, cpt, "pairs");
-  *out = CopyPlan{sh, vec, items, copy_walk(num_pairs, cpt, items)};
-  return 0;
+  return too_many_items(num_pairs, num_segments, tile_chunks(max_page, out->sh.chunk(), vec),
+                        "pairs");
 }
 
 // Byte offset of the pair table after num_segments CopySeg entries.
@@ -2170,14 +2096,20 @@ void sort_pairs(PairDesc* a, int64_t n, bool by_dst, PairDesc* tmp) {
   if (from != a) std::copy(from, from + n, a);
 }
 
-void pack_copy_desc(char* h, size_t pair_offset, int32_t num_segments, void* const* src_bases,
-                    void* const* dst_bases, const int64_t* page_bytes, int64_t num_pairs,
-                    const int64_t* src_ids, const int64_t* dst_ids, int64_t order,
-                    PairDesc* tmp) {
+// The tables of a copy at h: segments, class by class as the walk takes them,
+// then pairs.
+void pack_copy_desc(char* h, size_t pair_offset, const CopyPlan& plan, int32_t num_segments,
+                    void* const* src_bases, void* const* dst_bases, const int64_t* page_bytes,
+                    int64_t num_pairs, const int64_t* src_ids, const int64_t* dst_ids,
+                    int64_t order, PairDesc* tmp) {
+  const CopyLayout& l = plan.lay;
   CopySeg* hs = reinterpret_cast<CopySeg*>(h);
-  for (int32_t s = 0; s < num_segments; ++s)
-    hs[s] = CopySeg{static_cast<const char*>(src_bases[s]), static_cast<char*>(dst_bases[s]),
-                    page_bytes[s], 0};
+  for (int k = 0; k <= static_cast<int>(l.num_classes); ++k)
+    for (int32_t s = 0; s < num_segments; ++s)
+      if (l.num_classes == 0 ||
+          l.class_of(tile_chunks(page_bytes[s], plan.sh.chunk(), plan.vec)) == k)
+        *hs++ = CopySeg{static_cast<const char*>(src_bases[s]), static_cast<char*>(dst_bases[s]),
+                        page_bytes[s], 0};
   PairDesc* hp = reinterpret_cast<PairDesc*>(h + pair_offset);
   for (int64_t i = 0; i < num_pairs; ++i) hp[i] = PairDesc{src_ids[i], dst_ids[i]};
   // Targets are distinct and never sources, so any order gives the same
@@ -2200,15 +2132,15 @@ struct CopyKind {
 // device at `dv`, with the copy's grid and LDS policy.
 hipError_t copy_launch(const CopyPlan& p, const Tunables& t, int num_cus, int32_t num_segments,
                        const char* dv, hipStream_t stream, const CopyKind& kind = CopyKind()) {
-  const int64_t grid = launch_grid(t.copy_wgs_per_cu * num_cus, p.items, p.sh.wg);
+  const int64_t grid = launch_grid(t.copy_wgs_per_cu * num_cus, p.lay.walk.num_items, p.sh.wg);
   const unsigned lds = p.sh.wg == 1024 && p.sh.chunk() >= (int64_t(32) << 10)
                            ? static_cast<unsigned>(t.copy_lds_bytes) : 0u;
   const CopySeg* segs = reinterpret_cast<const CopySeg*>(dv);
   const PairDesc* pairs = reinterpret_cast<const PairDesc*>(dv + copy_pair_offset(num_segments));
   if (kind.probe)
     return launch_probe(p.sh, kind.probe, t.nt_stores != 0, grid, lds, stream, segs, pairs,
-                        p.walk, kind.sink, kind.magic);
-  return launch_copy(p.sh, p.vec, t.nt_stores != 0, grid, lds, stream, segs, pairs, p.walk,
+                        p.lay, kind.sink, kind.magic);
+  return launch_copy(p.sh, p.vec, t.nt_stores != 0, grid, lds, stream, segs, pairs, p.lay,
                      kind.guard);
 }
 
@@ -2219,20 +2151,22 @@ int copy_inline(const CopyPlan& p, const Tunables& t, int num_cus, int32_t num_s
                 void* const* src_bases, void* const* dst_bases, const int64_t* page_bytes,
                 int64_t num_pairs, const int64_t* src_ids, const int64_t* dst_ids,
                 hipStream_t stream, bool* launched) {
-  const size_t pair_offset = sizeof(CopySeg) * static_cast<size_t>(num_segments);
+  const size_t class_offset = sizeof(CopySeg) * static_cast<size_t>(num_segments);
+  const size_t pair_offset = class_offset + sizeof(CopyClass) * p.lay.num_classes;
   *launched = false;
   if (p.sh.u != 1 || p.sh.wg > 256 || (!p.vec && p.sh.wg != 64) ||
       pair_offset >= kInlineBytes ||
       num_pairs > static_cast<int64_t>((kInlineBytes - pair_offset) / sizeof(PairDesc)))
     return 0;
   InlineCopy a;
-  a.walk = p.walk;
+  a.walk = p.lay.walk;
   a.pair_offset = static_cast<uint32_t>(pair_offset);
-  a.pad[0] = a.pad[1] = 0;
+  a.num_classes = p.lay.num_classes;
   PairDesc tmp[kInlineBytes / sizeof(PairDesc)];
-  pack_copy_desc(reinterpret_cast<char*>(a.data), pair_offset, num_segments, src_bases, dst_bases,
-                 page_bytes, num_pairs, src_ids, dst_ids, t.copy_order, tmp);
-  const int64_t grid = launch_grid(t.copy_wgs_per_cu * num_cus, p.items, p.sh.wg);
+  pack_copy_desc(reinterpret_cast<char*>(a.data), pair_offset, p, num_segments, src_bases,
+                 dst_bases, page_bytes, num_pairs, src_ids, dst_ids, t.copy_order, tmp);
+  std::memcpy(a.data + class_offset, p.lay.classes.at, sizeof(CopyClass) * p.lay.num_classes);
+  const int64_t grid = launch_grid(t.copy_wgs_per_cu * num_cus, p.lay.walk.num_items, p.sh.wg);
   const hipError_t e = launch_inline(p.sh.wg, p.vec, t.nt_stores != 0, grid, stream, a);
   if (e != hipSuccess) return hip_fail(e, "copy_blocks_inline_kernel launch");
   *launched = true;
@@ -2256,7 +2190,7 @@ int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bas
                 "16 B multiples");
   const Tunables t = tunables();
   CopyPlan plan;
-  rc = copy_plan(t, vec, max_page, true, num_segments, num_pairs, &plan);
+  rc = copy_plan(t, vec, page_bytes, max_page, true, num_segments, num_pairs, &plan);
   if (rc) return rc;
   rc = copy_check_device(num_segments, src_bases, dst_bases, page_bytes, src_num_blocks,
                          dst_num_blocks, same_cache);
@@ -2267,7 +2201,7 @@ int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bas
   rc = get_ctx(&ctx);
   if (rc) return rc;
   if (!stream_has_all_cus(stream, ctx->num_cus))
-    rc = copy_plan(t, vec, max_page, false, num_segments, num_pairs, &plan);
+    rc = copy_plan(t, vec, page_bytes, max_page, false, num_segments, num_pairs, &plan);
   if (rc) return rc;
   if (!kind.probe && !kind.guard) {
     bool launched = false;
@@ -2282,7 +2216,7 @@ int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bas
   if (rc) return rc;
   char* h = ctx->ring.host + desc.off;
   std::vector<PairDesc> tmp(t.copy_order != 0 ? static_cast<size_t>(num_pairs) : 0);
-  pack_copy_desc(h, copy_pair_offset(num_segments), num_segments, src_bases, dst_bases,
+  pack_copy_desc(h, copy_pair_offset(num_segments), plan, num_segments, src_bases, dst_bases,
                  page_bytes, num_pairs, src_ids, dst_ids, t.copy_order, tmp.data());
   CopyKind launch = kind;
   rc = desc_stage(ctx->ring, desc, kind.guard, &launch.guard, stream);
@@ -2425,7 +2359,7 @@ int copy_noalloc(int32_t num_segments, void* const* bases, const int64_t* page_b
   if (rc || num_pairs == 0) return rc;
   const Tunables t = tunables();
   CopyPlan plan;
-  rc = copy_plan(t, vec, max_page, true, num_segments, num_pairs, &plan);
+  rc = copy_plan(t, vec, page_bytes, max_page, true, num_segments, num_pairs, &plan);
   if (rc) return rc;
   rc = copy_check_device(num_segments, bases, bases, page_bytes, num_blocks, num_blocks, true);
   if (rc) return rc;
@@ -2436,13 +2370,13 @@ int copy_noalloc(int32_t num_segments, void* const* bases, const int64_t* page_b
   rc = noalloc_scratch(dev, stream, &dv, &num_cus);
   if (rc) return rc;
   if (!stream_has_all_cus(stream, num_cus))
-    rc = copy_plan(t, vec, max_page, false, num_segments, num_pairs, &plan);
+    rc = copy_plan(t, vec, page_bytes, max_page, false, num_segments, num_pairs, &plan);
   if (rc) return rc;
   bool launched = false;
   rc = copy_inline(plan, t, num_cus, num_segments, bases, bases, page_bytes, num_pairs, src_ids,
                    dst_ids, stream, &launched);
   if (rc || launched) return rc;
-  pack_copy_desc(reinterpret_cast<char*>(g_noalloc_host), copy_pair_offset(num_segments),
+  pack_copy_desc(reinterpret_cast<char*>(g_noalloc_host), copy_pair_offset(num_segments), plan,
                  num_segments, bases, bases, page_bytes, num_pairs, src_ids, dst_ids,
                  t.copy_order, g_noalloc_order);
   // The descriptor reaches `scratch` through kernel arguments, not a copy

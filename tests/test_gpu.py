@@ -682,6 +682,94 @@ def test_copy_walk_covers_every_item_once(gpu, page, segs, pairs):
         assert torch.equal(o[d], t[s]) and int((o != 0).any(1).sum()) <= pairs
 
 
+_K = 1024
+
+
+@pytest.mark.parametrize("pages", [
+    [160 * _K, 16 * _K], [16 * _K, 160 * _K, 512], [2048 * _K] + [16 * _K] * 7,
+    [41984, 8448, 8448, 41984], [4096, 4096, 16, 8192, 4096], [20484, 1028, 33, 1],
+    [16 * _K * k for k in (1, 9, 2, 8, 3, 7, 4, 6, 5, 10)], [16400, 4096, 64 * _K],
+    [1000 + 16 * ((k * 37) % 71) for k in range(70)] + [80 * k for k in range(1, 50)],
+], ids=lambda p: f"{len(p)}x{p[0]}")
+@pytest.mark.parametrize("pairs", [1, 27, 300])
+def test_copies_of_mixed_pages(gpu, restore_tuning, pages, pairs):
+    """Caches whose tensors have pages of several sizes, as many as the walk
+    tells apart and more, aligned and not: every entry point, on the whole
+    chip and on a masked stream, and the loads-per-lane shapes."""
+    _say("mixed pages", len(pages), pages[0], pairs)
+    if sum(pages) * pairs > 400 << 20:
+        pairs = (400 << 20) // sum(pages)
+    g = torch.Generator(device=gpu).manual_seed(pairs)
+    n = 2 * pairs + 3
+    ids = np.random.default_rng(pairs).permutation(n)
+    src, dst = ids[:pairs], ids[pairs:2 * pairs]
+    start = [torch.randint(0, 256, (n, p), dtype=torch.uint8, device=gpu, generator=g)
+             for p in pages]
+    s, d = torch.from_numpy(src.copy()).to(gpu), torch.from_numpy(dst.copy()).to(gpu)
+    want = [t.clone().index_copy_(0, d, t[s]) for t in start]
+    masked = ops.DedicatedStream(gpu, ops.xcd_cu_mask(8, device=gpu))
+
+    def check(what, entry, **kw):
+        got = [t.clone() for t in start]
+        torch.cuda.synchronize()
+        entry(got, src, dst, **kw)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), what
+
+    try:
+        for entry in (ops.copy_blocks, ops.copy_blocks_noalloc):
+            check(entry.__name__, entry)
+            check((entry.__name__, "masked"), entry, stream=masked.stream)
+        other = [torch.zeros_like(t) for t in start]
+        ops.migrate_blocks(start, other, src, dst)
+        torch.cuda.synchronize()
+        for t, o, w in zip(start, other, want):
+            assert torch.equal(o[d], w[d]) and int((o != 0).any(1).sum()) <= pairs
+        for unroll in (1, 10):
+            _lib.tune(_lib.TUNE_COPY_UNROLL, unroll)
+            check(("unroll", unroll), ops.copy_blocks)
+    finally:
+        masked.close()
+
+
+@pytest.mark.parametrize("n_seg,sizes,n", [(72, 2, 92), (72, 2, 93), (72, 8, 80), (72, 8, 81),
+                                           (111, 8, 1), (117, 2, 2), (117, 2, 3), (118, 2, 1)])
+def test_mixed_pages_around_a_launch_s_arguments(gpu, n_seg, sizes, n):
+    """A launch's arguments hold 3808 bytes: 32 a segment, 32 for each page
+    size behind the first, 16 a pair."""
+    _say("mixed pages in a launch's arguments", n_seg, sizes, n)
+    pages = [4096 * (1 + i % sizes) for i in range(n_seg)]
+    g = torch.Generator(device=gpu).manual_seed(n)
+    blocks = 2 * n + 1
+    ids = np.random.default_rng(n_seg).permutation(blocks)
+    src, dst = ids[:n], ids[n:2 * n]
+    start = [torch.randint(0, 256, (blocks, p), dtype=torch.uint8, device=gpu, generator=g)
+             for p in pages]
+    s, d = torch.from_numpy(src.copy()).to(gpu), torch.from_numpy(dst.copy()).to(gpu)
+    want = [t.clone().index_copy_(0, d, t[s]) for t in start]
+    for entry in (ops.copy_blocks, ops.copy_blocks_noalloc):
+        got = [t.clone() for t in start]
+        entry(got, src, dst)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), entry.__name__
+
+
+def test_copy_probes_over_mixed_pages(gpu):
+    """The probes walk the copy's items: every target tile of every size is
+    written once over, and nothing else."""
+    pages = [160 * _K, 512, 16 * _K, 4096, 16]
+    segs = [torch.zeros(20, p, dtype=torch.uint8, device=gpu) for p in pages]
+    ids = np.random.default_rng(3).permutation(20)
+    sink = torch.zeros(4, dtype=torch.int32, device=gpu)
+    ops.copy_probe(ops.PROBE_WRITE, segs, ids[:9], ids[9:18], sink, magic=0x01020304)
+    torch.cuda.synchronize()
+    d = torch.from_numpy(ids[9:18].copy()).to(gpu)
+    for t, p in zip(segs, pages):
+        words = t.view(torch.int32).view(20, p // 16, 4)
+        assert bool((words[d][:, :, 3] == 0x01020304).all())
+        assert int((t != 0).any(1).sum()) == 9
+
+
 @pytest.mark.parametrize("order", [0, 1, 2])
 def test_copy_blocks_pair_orders_vs_oracle(gpu, oracle, restore_tuning, order):
     """The library may hand the kernel the pairs in the caller's order, by
