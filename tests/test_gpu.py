@@ -682,6 +682,39 @@ def test_copy_walk_covers_every_item_once(gpu, page, segs, pairs):
         assert torch.equal(o[d], t[s]) and int((o != 0).any(1).sum()) <= pairs
 
 
+@pytest.mark.parametrize("workgroups,unroll", [(1, 2), (31, 4), (32, 4), (63, 2), (64, 2), (65, 2),
+                                               (128, 1), (127, 1)])
+def test_persistent_grids_around_the_wait_for_stores(gpu, restore_tuning, workgroups, unroll):
+    """From 512 KiB in flight the workgroups of swaps and weight loads wait
+    for an item's stores before they load the next; the bytes are the same on
+    both sides of that line, in whole items and tails, aligned or not."""
+    _say("persistent grids", workgroups, unroll)
+    for key in (_lib.TUNE_SWAP_OUT_WORKGROUPS, _lib.TUNE_SWAP_IN_WORKGROUPS):
+        _lib.tune(key, workgroups)
+    _lib.tune(_lib.TUNE_SWAP_UNROLL, unroll)
+    g = torch.Generator(device=gpu).manual_seed(workgroups)
+    for page in (33 * 1024 + 16, 16 * 1024, 9001):
+        n = 30
+        cache = torch.randint(0, 256, (2 * n, page), dtype=torch.uint8, device=gpu, generator=g)
+        start = cache.clone()
+        pool = ops.PinnedHostPool(n * page)
+        ids = np.random.default_rng(page).permutation(2 * n)
+        out, back = ids[:n], ids[n:]
+        slots = np.arange(n)
+        ops.swap(out, slots, False, cache, pool.tensor.view(n, page))
+        ops.swap(slots, back, True, cache, pool.tensor.view(n, page))
+        loaded = torch.empty(n * page, dtype=torch.uint8, device=gpu)
+        cuts = [0, 5, 20000, 20016, n * page]
+        ops.load_slices([loaded[a:b] for a, b in zip(cuts, cuts[1:])],
+                        [pool.tensor[a:b] for a, b in zip(cuts, cuts[1:])])
+        torch.cuda.synchronize()
+        o, b = torch.from_numpy(out.copy()).to(gpu), torch.from_numpy(back.copy()).to(gpu)
+        assert torch.equal(pool.tensor.view(n, page), start[o].cpu())
+        assert torch.equal(cache, start.index_copy(0, b, start[o]))
+        assert torch.equal(loaded, start[o].view(-1))
+        torch.cuda.synchronize()
+
+
 _K = 1024
 
 
