@@ -29,6 +29,7 @@
 #include "aegkv.h"
 #include "copy_walk.h"
 #include "errors.h"
+#include "staged_runs.h"
 
 #include <algorithm>
 #include <cstdarg>
@@ -1330,31 +1331,6 @@ hipError_t launch_slices(bool vec, bool nt, int64_t grid, hipStream_t st,
 
 // ------------------------------------------------------------ swap core --
 
-struct SwapLayout {
-  int32_t num_segments;
-  void* const* bases;
-  const int64_t* page_bytes;
-  const int64_t* host_offsets;
-  const uint64_t* owner_masks;
-  int64_t device_num_blocks;
-  int32_t num_groups;
-  const int64_t* kpp;
-  char* host_pool;
-  int64_t host_num_blocks;
-  int64_t host_page_bytes;
-  int64_t host_rank_offset;
-};
-
-struct SwapList {
-  int64_t n;
-  const int64_t* src;
-  const int64_t* dst;
-  const int32_t* group;     // may be null: all group 0
-  const int64_t* first;     // may be null: all 0
-  const int64_t* valid;     // may be null: all kpp[group]
-  const uint64_t* guard;    // may be null: the kernels move nothing once *guard != 0
-};
-
 bool mul_fits(int64_t a, int64_t b) { return a >= 0 && b >= 0 && (b == 0 || a <= INT64_MAX / b); }
 
 // Argument checks that need no HIP call (run first, so a bad argument costs
@@ -1479,12 +1455,6 @@ ShapeSel swap_shape(const Tunables& t, bool vec, int64_t max_page) {
                            : ShapeSel{256, static_cast<int>(t.swap_unroll)};
 }
 
-struct Run {
-  int64_t host_off;   // byte offset inside the host pool
-  int64_t stage_off;  // byte offset inside staging
-  int64_t len;
-};
-
 // The tables of a swap of entries order[lo, hi), at h: segments, then kernel
 // blocks per page, then entries resolved to the given host side.
 void pack_swap_desc(char* h, size_t kpp_off, size_t ent_off, const SwapLayout& L,
@@ -1593,66 +1563,6 @@ int enqueue_swap_kernel(DeviceCtx* ctx, const SwapLayout& L, const SwapList& E,
 
 // A staged chunk with more host runs than this counts as scattered.
 constexpr size_t kManyRuns = 16;
-
-// Runs of host bytes one staged entry moves, merged when contiguous.
-void entry_runs(const SwapLayout& L, const SwapList& E, int64_t i, bool is_swap_in,
-                int64_t slot, int64_t composite, std::vector<Run>& runs) {
-  const int32_t g = E.group ? E.group[i] : 0;
-  const int64_t k = L.kpp[g];
-  const int64_t first = E.first ? E.first[i] : 0;
-  const int64_t valid = E.valid ? E.valid[i] : k;
-  const int64_t host_id = is_swap_in ? E.src[i] : E.dst[i];
-  const int64_t host_page = host_id * L.host_page_bytes + L.host_rank_offset;
-  const int64_t stage_page = slot * composite;
-  for (int32_t s = 0; s < L.num_segments; ++s) {
-    if (!((L.owner_masks[s] >> g) & 1ull)) continue;
-    const int64_t unit = L.page_bytes[s] / k;
-    const int64_t off = unit * first, len = unit * valid;
-    if (len == 0) continue;
-    const int64_t ho = host_page + L.host_offsets[s] + off;
-    const int64_t so = stage_page + L.host_offsets[s] + off;
-    if (!runs.empty()) {
-      Run& r = runs.back();
-      if (r.host_off + r.len == ho && r.stage_off + r.len == so) {
-        r.len += len;
-        continue;
-      }
-    }
-    runs.push_back({ho, so, len});
-  }
-}
-
-// The runs of a staged chunk, order[lo, hi), in staging slots of their own.
-void chunk_runs(const SwapLayout& L, const SwapList& E, const std::vector<int64_t>& order,
-                size_t lo, size_t hi, bool is_swap_in, int64_t composite,
-                std::vector<Run>& runs) {
-  runs.clear();
-  for (size_t j = lo; j < hi; ++j)
-    entry_runs(L, E, order[j], is_swap_in, static_cast<int64_t>(j - lo), composite, runs);
-}
-
-// How a STAGED call's runs move, by the runs of its first chunk.
-//
-// The runtime takes 3-7 us a copy, over two streams, so runs below 128 KiB on
-// average stay under a third of the link rate: such calls go out as the
-// DIRECT kernel. 480 runs of 9 KiB: 1315 us staged, 81 direct; 60 blocks of
-// 40 KiB, some adjacent: 229 and 47. Longer runs stay staged, which leaves
-// the CUs alone.
-//
-// Up to four runs in one chunk leave nothing to overlap, so their copies go
-// on the caller's stream, without the events that fork to the library's
-// streams and back (20-40 us): one run of 9.4 MB 265 -> 225 us, of 47 MB 942
-// -> 907, of 2.5 MB 166 -> 103, and with several callers in turn, where the
-// runtime moves some copies at 29 GB/s, of 472 MB 10.4 -> 9.15 ms. Four runs
-// of 2.4 MB 272 -> 254 us, twenty 1002 -> 1058.
-constexpr int64_t kShortRun = int64_t(128) << 10;
-constexpr size_t kFewRuns = 4;
-
-bool runs_are_short(const std::vector<Run>& runs) {
-  int64_t bytes = 0;
-  for (const Run& r : runs) bytes += r.len;
-  return runs.size() > kFewRuns && bytes < kShortRun * static_cast<int64_t>(runs.size());
-}
 
 // A stream on a hardware queue of its own: a stream created with a CU mask
 // gets a dedicated queue (here the mask enables every CU), while plain
@@ -1899,16 +1809,17 @@ int swap_core(const SwapLayout& L, const SwapList& E, bool is_swap_in, int mode,
   rc = validate_list(L, E, is_swap_in);
   if (rc) return rc;
   if (E.n == 0) return 0;
-  {
-    // the whole list in one launch (a staged chunk holds fewer entries)
-    int64_t max_page = 0;
-    for (int32_t s = 0; s < L.num_segments; ++s) max_page = std::max(max_page, L.page_bytes[s]);
-    const bool vec = staged ? dev_vec && composite % 16 == 0 : dev_vec && host_vec;
-    const ShapeSel sh = swap_shape(t, vec, max_page);
-    const int64_t cpt = (max_page + sh.chunk() - 1) / sh.chunk();
-    if (launch_items(E.n, L.num_segments, cpt) < 0)
-      return too_many_items(E.n, L.num_segments, cpt, "entries");
-  }
+  int64_t max_page = 0;
+  for (int32_t s = 0; s < L.num_segments; ++s) max_page = std::max(max_page, L.page_bytes[s]);
+  auto chunks = [&](bool vec) {
+    const int64_t chunk = swap_shape(t, vec, max_page).chunk();
+    return (max_page + chunk - 1) / chunk;
+  };
+  // the whole list in one launch (a staged chunk holds fewer entries)
+  const int64_t cpt = chunks(dev_vec && (staged ? composite % 16 == 0 : host_vec));
+  if (launch_items(E.n, L.num_segments, cpt) < 0)
+    return too_many_items(E.n, L.num_segments, cpt, "entries");
+  const bool direct_fits = launch_items(E.n, L.num_segments, chunks(dev_vec && host_vec)) >= 0;
   rc = check_layout_pointers(L);
   if (rc) return rc;
   rc = refuse_capture(stream);
@@ -1940,11 +1851,14 @@ int swap_core(const SwapLayout& L, const SwapList& E, bool is_swap_in, int mode,
       std::max<int64_t>(1, std::min<int64_t>(E.n, t.staging_bytes / composite)));
   std::vector<Run> runs;
   chunk_runs(L, E, order, 0, step, is_swap_in, composite, runs);
-  if (t.staged_short_runs && runs_are_short(runs)) return direct();
+  if (t.staged_short_runs && direct_fits &&
+      cheap_as_direct(order.size() <= step ? run_totals(runs)
+                                           : call_runs(L, E, order, is_swap_in, composite, step)))
+    return direct();
   // Staging comes from hipMallocAsync (256 B aligned) with a composite stride.
   const bool vec_stage = dev_vec && composite % 16 == 0;
   int k = static_cast<int>(std::min<int64_t>(t.staged_dma_streams, kMaxDmaStreams));
-  if (order.size() <= step && runs.size() <= kFewRuns) k = 0;
+  if (order.size() <= step && static_cast<int64_t>(runs.size()) <= kFewRuns) k = 0;
   const bool overlap = (t.staged_overlap >> (is_swap_in ? 1 : 0)) & 1;
   if (k <= 1 || !overlap)
     return staged_serial(ctx, L, E, order, is_swap_in, composite, step, runs, vec_stage, t, k,

@@ -62,8 +62,10 @@ extern "C" {
                                staging, plus hipMemcpyAsync of merged runs
                                (the runtime runs them on SDMA engines or as
                                blit kernels); leaves the CUs to concurrent
-                               compute. A call whose host runs are short goes
-                               DIRECT (AEGKV_TUNE_STAGED_SHORT_RUNS)           */
+                               compute. A call whose host runs are short and
+                               few bytes in all goes DIRECT, which takes no
+                               more from compute beside it
+                               (AEGKV_TUNE_STAGED_SHORT_RUNS)                  */
 
 /* Environment, read once per process before the first call:
  *   AEGKV_AUTO_D2H, AEGKV_AUTO_H2D = direct | staged   (what AUTO picks)
@@ -112,10 +114,11 @@ extern "C" {
                                         as given (0), sorted by target id
                                         (1, default) or by source id (2);
                                         the result does not depend on it   */
-#define AEGKV_TUNE_STAGED_SHORT_RUNS 19 /* 1 (default): a STAGED swap whose
-                                        host runs are below 128 KiB on
-                                        average (more than 4 of them) moves
-                                        as DIRECT; 0: always staged        */
+#define AEGKV_TUNE_STAGED_SHORT_RUNS 19 /* 1 (default): a STAGED swap (asked
+                                        for or by AUTO) of more than 4 host
+                                        runs, below 128 KiB on average and at
+                                        most 2 MiB + 16 KiB a run in all,
+                                        moves as DIRECT; 0: always staged  */
 
 /* ABI version of the loaded library (AEGKV_ABI_VERSION). */
 int aegkv_abi_version(void);

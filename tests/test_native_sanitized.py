@@ -1,8 +1,9 @@
 """Host code of libaegkv under AddressSanitizer and UndefinedBehaviorSanitizer
 (CPU only): the native planner (aegaeon_amd/csrc/plan.cpp) driven with
-random block tables by tests/native/plan_fuzz.cpp, and the walk of a block
-copy (aegaeon_amd/csrc/copy_walk.h) enumerated by
-tests/native/copy_walk_check.cpp."""
+random block tables by tests/native/plan_fuzz.cpp, the walk of a block copy
+(aegaeon_amd/csrc/copy_walk.h) enumerated by tests/native/copy_walk_check.cpp,
+and the runs of STAGED swaps (aegaeon_amd/csrc/staged_runs.h) counted by
+tests/native/staged_runs_check.cpp."""
 
 import shutil
 import subprocess
@@ -13,21 +14,32 @@ import pytest
 REPO = Path(__file__).resolve().parent.parent
 
 
-@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ is not installed")
-def test_copy_walk_covers_every_byte_once(tmp_path):
-    """One page size, several and more than the walk tells apart, at any
-    alignment: every byte of every tile in exactly one item, and no items
-    launched for nothing where the sizes are up to eight."""
-    exe = tmp_path / "copy_walk_check"
+def _run_native_check(tmp_path, name):
+    """Build tests/native/<name>.cpp with sanitizers and run it."""
+    exe = tmp_path / name
     cmd = ["g++", "-std=c++17", "-O1", "-g", "-fno-omit-frame-pointer", "-Wall",
            "-fsanitize=address,undefined", "-fno-sanitize-recover=all",
            f"-I{REPO / 'aegaeon_amd' / 'csrc'}",
-           str(REPO / "tests" / "native" / "copy_walk_check.cpp"), "-o", str(exe)]
+           str(REPO / "tests" / "native" / f"{name}.cpp"), "-o", str(exe)]
     res = subprocess.run(cmd, capture_output=True, text=True, timeout=300)
     assert res.returncode == 0, res.stderr
     run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     assert run.returncode == 0, run.stdout + run.stderr
     assert "clean" in run.stdout
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ is not installed")
+def test_copy_walk_covers_every_byte_once(tmp_path):
+    """One page size, several and more than the walk tells apart, at any
+    alignment: every byte of every tile in exactly one item, and no items
+    launched for nothing where the sizes are up to eight."""
+    _run_native_check(tmp_path, "copy_walk_check")
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ is not installed")
+def test_staged_calls_are_judged_by_all_their_runs(tmp_path):
+    """Whether a STAGED swap goes DIRECT depends on every chunk's runs."""
+    _run_native_check(tmp_path, "staged_runs_check")
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="g++ is not installed")

@@ -1,6 +1,6 @@
-"""STAGED swaps by the runs of host bytes they leave: calls of short runs move
-as DIRECT, calls of a few runs copy on the caller's stream, the others fork
-over the library's streams. All give the same bytes.
+"""STAGED swaps by the runs of host bytes they leave: calls of short runs, few
+bytes in all, move as DIRECT, calls of a few runs copy on the caller's stream,
+the others fork over the library's streams. All give the same bytes.
 """
 
 import sys
@@ -36,13 +36,14 @@ def test_the_rule_is_on_and_takes_0_or_1():
 
 
 # page, entries, host ids, staging bytes: runs of one page each (no two host
-# pages adjacent), around 128 KiB and around four of them; adjacent pages that
-# merge; and more than one chunk
+# pages adjacent), around 128 KiB, around four of them and around 2 MiB + 16 KiB
+# a run; adjacent pages that merge; and more than one chunk
 @pytest.mark.parametrize("page,n,step,staging", [
     (128 << 10, 4, 2, None), (128 << 10, 5, 2, None), ((128 << 10) - 16, 4, 2, None),
     ((128 << 10) - 16, 5, 2, None), ((128 << 10) + 16, 5, 2, None), (4096, 1, 1, None),
     (4096, 40, 1, None), (4099, 7, 2, None), (256 << 10, 9, 2, 1 << 20), (256 << 10, 9, 1, 1 << 20),
     (20 << 10, 120, 2, 1 << 20), (300 << 10, 4, 1, 1 << 20),
+    (32 << 10, 128, 2, None), (32 << 10, 129, 2, None), (32 << 10, 128, 2, 1 << 20),
 ])
 @pytest.mark.parametrize("rule", [1, 0])
 @pytest.mark.parametrize("uncached", [False, True])
