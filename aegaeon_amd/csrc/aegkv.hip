@@ -476,6 +476,7 @@ __global__ __launch_bounds__(WG) void swap_tiles_kernel(
 // behind the transfers (100-200 us a time), a launch's packet and a staged
 // descriptor among them, so a launch less counts double there.
 constexpr uint32_t kInlineSwapBytes = 3776;
+typedef __attribute__((address_space(4))) const char kernarg_char;
 struct alignas(16) InlineSwap {
   SwapWalk walk;
   uint32_t kpp_offset, ent_offset;
@@ -485,7 +486,6 @@ struct alignas(16) InlineSwap {
 };
 static_assert(offsetof(InlineSwap, data) % 16 == 0 && sizeof(InlineSwap) <= 3840,
               "InlineSwap layout: 4 KiB of arguments, 256 bytes of them hidden ones");
-typedef __attribute__((address_space(4))) const char kernarg_char;
 
 template <bool TO_HOST, bool VEC, bool NT_STORE>
 __global__ __launch_bounds__(256) void swap_inline_kernel(InlineSwap a) {
@@ -500,11 +500,22 @@ __global__ __launch_bounds__(256) void swap_inline_kernel(InlineSwap a) {
                                              (kernarg_i64*)(data + a.kpp_offset), a.walk);
 }
 
-// The classes of a walk where the launch put them: the kernel's first
-// argument. Indexed as a parameter they would be copied to scratch memory.
+// The classes of a walk where the launch put them. Indexed as a parameter they
+// would be copied to scratch memory. They come last of the arguments, so that
+// all a cache with one page size needs lies in one line of 64 bytes: behind
+// them, on a line border, copies of 0.6-4 ms took 1-3 us longer.
+struct CopyArgs {
+  const CopySeg* segs;
+  const PairDesc* pairs;
+  CopyWalk walk;
+  const uint64_t* guard;  // a probe's sink and magic
+  CopyClasses classes;
+};
+static_assert(offsetof(CopyArgs, classes) == 64, "CopyArgs layout");
 typedef __attribute__((address_space(4))) const CopyClass kernarg_class;
-__device__ __forceinline__ kernarg_class* first_argument() {
-  return (kernarg_class*)__builtin_amdgcn_kernarg_segment_ptr();
+__device__ __forceinline__ kernarg_class* argument_classes() {
+  return (kernarg_class*)((kernarg_char*)__builtin_amdgcn_kernarg_segment_ptr() +
+                          offsetof(CopyArgs, classes));
 }
 
 // copy_blocks: one item is one chunk of one (segment, pair) tile. The host
@@ -512,10 +523,10 @@ __device__ __forceinline__ kernarg_class* first_argument() {
 template <int WG, int U, bool VEC, bool NT_STORE, typename Segs, typename Pairs,
           typename Classes>
 __device__ __forceinline__ void copy_items(Segs segs, Pairs pairs, const CopyWalk& walk,
-                                           Classes classes, uint32_t num_classes) {
+                                           Classes classes) {
   constexpr int64_t kChunk = Shape<WG, U>::kChunk;
   for (uint32_t w = blockIdx.x; w < walk.num_items; w += gridDim.x) {
-    const CopyItem it = copy_item(walk, classes, num_classes, w);
+    const CopyItem it = copy_item(walk, classes, w);
     const int64_t src_block = pairs[it.pair].src, dst_block = pairs[it.pair].dst;
     const int64_t page = segs[it.segment].page_bytes;
     const char* src = segs[it.segment].src + src_block * page;
@@ -537,13 +548,13 @@ __device__ __forceinline__ void copy_items(Segs segs, Pairs pairs, const CopyWal
 }
 
 template <int WG, int U, bool VEC, bool NT_STORE>
-__global__ __launch_bounds__(WG) void copy_blocks_kernel(CopyClasses, uint32_t num_classes,
-                                                         const CopySeg* __restrict__ segs,
+__global__ __launch_bounds__(WG) void copy_blocks_kernel(const CopySeg* __restrict__ segs,
                                                          const PairDesc* __restrict__ pairs,
                                                          CopyWalk walk,
-                                                         const uint64_t* __restrict__ guard) {
+                                                         const uint64_t* __restrict__ guard,
+                                                         CopyClasses) {
   if (guard_set(guard)) return;
-  copy_items<WG, U, VEC, NT_STORE>(segs, pairs, walk, first_argument(), num_classes);
+  copy_items<WG, U, VEC, NT_STORE>(segs, pairs, walk, argument_classes());
 }
 
 // A short copy's whole descriptor (segment table, classes of the walk behind
@@ -559,8 +570,7 @@ __global__ __launch_bounds__(WG) void copy_blocks_kernel(CopyClasses, uint32_t n
 constexpr uint32_t kInlineBytes = 3808;
 struct alignas(16) InlineCopy {
   CopyWalk walk;
-  uint32_t pair_offset;  // bytes of the segment table and the classes
-  uint32_t num_classes;
+  uint32_t class_offset, pair_offset;  // from data
   unsigned char data[kInlineBytes];
 };
 static_assert(offsetof(InlineCopy, data) == 32 && sizeof(InlineCopy) <= 4096,
@@ -574,9 +584,8 @@ __global__ __launch_bounds__(WG) void copy_blocks_inline_kernel(InlineCopy a) {
   // only argument and starts its argument segment
   kernarg_char* data =
       (kernarg_char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(InlineCopy, data);
-  kernarg_char* pairs = data + a.pair_offset;
-  copy_items<WG, 1, VEC, NT_STORE>((kernarg_seg*)data, (kernarg_pair*)pairs, a.walk,
-                                   (kernarg_class*)pairs - a.num_classes, a.num_classes);
+  copy_items<WG, 1, VEC, NT_STORE>((kernarg_seg*)data, (kernarg_pair*)(data + a.pair_offset),
+                                   a.walk, (kernarg_class*)(data + a.class_offset));
 }
 
 // Measurement twins of copy_blocks_kernel (aegkv_copy_probe): the same
@@ -590,17 +599,16 @@ constexpr int PROBE_READ = 1;
 constexpr int PROBE_WRITE = 2;
 
 template <int WG, int U, int KIND, bool NT_STORE>
-__global__ __launch_bounds__(WG) void copy_probe_kernel(CopyClasses, uint32_t num_classes,
-                                                        const CopySeg* __restrict__ segs,
+__global__ __launch_bounds__(WG) void copy_probe_kernel(const CopySeg* __restrict__ segs,
                                                         const PairDesc* __restrict__ pairs,
                                                         CopyWalk walk, uint32_t* sink,
-                                                        uint32_t magic) {
+                                                        uint32_t magic, CopyClasses) {
   constexpr int64_t kChunk = Shape<WG, U>::kChunk;
   const uint32_t tid = threadIdx.x;
   v4u acc = {0u, 0u, 0u, 0u};
   const v4u pattern = {tid, blockIdx.x, 0x5a5a5a5au, magic};
   for (uint32_t w = blockIdx.x; w < walk.num_items; w += gridDim.x) {
-    const CopyItem it = copy_item(walk, first_argument(), num_classes, w);
+    const CopyItem it = copy_item(walk, argument_classes(), w);
     const PairDesc pr = pairs[it.pair];
     const CopySeg seg = segs[it.segment];
     const int64_t begin = static_cast<int64_t>(it.chunk) * kChunk;
@@ -1235,7 +1243,7 @@ hipError_t launch_copy_t(int64_t grid, unsigned lds, hipStream_t st, const CopyS
                          const PairDesc* p, const CopyLayout& l, const uint64_t* guard) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
   hipLaunchKernelGGL((copy_blocks_kernel<WG, U, VEC, NT>), dim3(static_cast<uint32_t>(grid)),
-                     dim3(WG), lds, st, l.classes, l.num_classes, s, p, l.walk, guard);
+                     dim3(WG), lds, st, s, p, l.walk, guard, l.classes);
   return hipGetLastError();
 }
 
@@ -1286,7 +1294,7 @@ hipError_t launch_probe_t(int64_t grid, unsigned lds, hipStream_t st, const Copy
                           uint32_t magic) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
   hipLaunchKernelGGL((copy_probe_kernel<WG, U, KIND, NT>), dim3(static_cast<uint32_t>(grid)),
-                     dim3(WG), lds, st, l.classes, l.num_classes, s, p, l.walk, sink, magic);
+                     dim3(WG), lds, st, s, p, l.walk, sink, magic, l.classes);
   return hipGetLastError();
 }
 
@@ -2105,8 +2113,8 @@ int copy_inline(const CopyPlan& p, const Tunables& t, int num_cus, int32_t num_s
     return 0;
   InlineCopy a;
   a.walk = p.lay.walk;
+  a.class_offset = static_cast<uint32_t>(class_offset);
   a.pair_offset = static_cast<uint32_t>(pair_offset);
-  a.num_classes = p.lay.num_classes;
   PairDesc tmp[kInlineBytes / sizeof(PairDesc)];
   pack_copy_desc(reinterpret_cast<char*>(a.data), pair_offset, p, num_segments, src_bases,
                  dst_bases, page_bytes, num_pairs, src_ids, dst_ids, t.copy_order, tmp);

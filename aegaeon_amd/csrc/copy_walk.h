@@ -81,7 +81,8 @@ inline int64_t tile_chunks(int64_t page, int64_t chunk, bool vec) {
 // number 2.66 -> 1.69 ms, 41,984 and 8,448 bytes 0.96 -> 0.79. A cache with
 // one page size pays one scalar comparison an item.
 struct alignas(32) CopyClass {
-  uint32_t first_item, first_segment, chunks_per_tile;
+  uint32_t first_item, end;
+  uint32_t first_segment, chunks_per_tile;
   uint32_t remap_end;  // counted from first_item, as the renumbering is
   uint32_t run_shift;
 };
@@ -104,28 +105,27 @@ struct CopyItem {
   uint32_t pair, segment, chunk, last;
 };
 
-// Item w. `classes`: the num_classes classes behind the first one.
-template <typename Classes>
-AEGKV_HOST_DEVICE CopyItem copy_item(const CopyWalk& k, Classes classes, uint32_t num_classes,
-                                     uint32_t w) {
-  uint32_t first_segment = 0;
-  uint32_t chunks = k.chunks_per_tile, remap_end = k.remap_end, shift = k.run_shift;
-  if (w >= k.first_end) {
-    uint32_t i = 0;
-    while (i + 1 < num_classes && w >= classes[i + 1].first_item) ++i;
-    w -= classes[i].first_item;
-    first_segment = classes[i].first_segment;
-    chunks = classes[i].chunks_per_tile;
-    remap_end = classes[i].remap_end;
-    shift = classes[i].run_shift;
-  }
+// Item w of a class, counted from its first.
+AEGKV_HOST_DEVICE CopyItem class_item(uint32_t num_pairs, uint32_t first_segment, uint32_t chunks,
+                                      uint32_t remap_end, uint32_t shift, uint32_t w) {
   if (w < remap_end) {
     const uint32_t r = w & ((8u << shift) - 1u);
     w = w - r + ((r & 7u) << shift) + (r >> 3);
   }
   const uint32_t tile = w / chunks;
-  const uint32_t s = tile / k.num_pairs;
-  return {tile - s * k.num_pairs, first_segment + s, w - tile * chunks, chunks - 1};
+  const uint32_t s = tile / num_pairs;
+  return {tile - s * num_pairs, first_segment + s, w - tile * chunks, chunks - 1};
+}
+
+// Item w (below num_items). `classes`: those behind the first one.
+template <typename Classes>
+AEGKV_HOST_DEVICE CopyItem copy_item(const CopyWalk& k, Classes classes, uint32_t w) {
+  if (w < k.first_end)
+    return class_item(k.num_pairs, 0, k.chunks_per_tile, k.remap_end, k.run_shift, w);
+  uint32_t i = 0;
+  while (w >= classes[i].end) ++i;
+  return class_item(k.num_pairs, classes[i].first_segment, classes[i].chunks_per_tile,
+                    classes[i].remap_end, classes[i].run_shift, w - classes[i].first_item);
 }
 
 // A walk as the host lays it out. The descriptor holds the segments class by
@@ -169,31 +169,39 @@ inline bool lay_walk(const int64_t* page_bytes, int32_t num_segments, int64_t nu
     }
     --n;
   };
+  int at = -1;  // the last segment's count
   for (int32_t s = 0; s < num_segments; ++s) {
+    if (at >= 0 && page_bytes[s] == page_bytes[s - 1]) {
+      ++segments[at];
+      continue;
+    }
     const int64_t c = tile_chunks(page_bytes[s], chunk, vec);
     if (launch_items(num_pairs, 1, c) < 0) return false;
-    int i = 0;
-    while (i < n && count[i] > c) ++i;
-    if (i == n || count[i] != c) {
-      for (int j = n; j > i; --j) {
+    at = 0;
+    while (at < n && count[at] > c) ++at;
+    if (at == n || count[at] != c) {
+      for (int j = n; j > at; --j) {
         count[j] = count[j - 1];
         segments[j] = segments[j - 1];
       }
-      count[i] = c;
-      segments[i] = 0;
+      count[at] = c;
+      segments[at] = 0;
       ++n;
     }
-    ++segments[i];
-    if (n > kSizes) merge();
+    ++segments[at];
+    if (n > kSizes) {
+      merge();
+      at = -1;
+    }
   }
   while (n > kCopyClasses) merge();
   out->num_classes = static_cast<uint32_t>(n - 1);
-  for (int i = 0; i < n; ++i) {
-    out->chunks[i] = count[i];
-    segments[i] = 0;
+  for (int i = 0; i < n; ++i) out->chunks[i] = count[i];
+  if (n > 1) {  // a joined size may have come again
+    for (int i = 0; i < n; ++i) segments[i] = 0;
+    for (int32_t s = 0; s < num_segments; ++s)
+      ++segments[out->class_of(tile_chunks(page_bytes[s], chunk, vec))];
   }
-  for (int32_t s = 0; s < num_segments; ++s)
-    ++segments[out->class_of(tile_chunks(page_bytes[s], chunk, vec))];
   int64_t items = 0, segment = 0;
   for (int i = 0; i < n; ++i) {
     const int64_t mine = launch_items(num_pairs, segments[i], count[i]);
@@ -201,12 +209,12 @@ inline bool lay_walk(const int64_t* page_bytes, int32_t num_segments, int64_t nu
     uint32_t shift = 5;
     while (shift < 20 && (int64_t(1) << shift) < 32 * count[i]) ++shift;
     const int64_t span = int64_t(8) << shift;
-    const CopyClass k{static_cast<uint32_t>(items), static_cast<uint32_t>(segment),
-                      static_cast<uint32_t>(count[i]), static_cast<uint32_t>(mine / span * span),
-                      shift};
+    const CopyClass k{static_cast<uint32_t>(items),   static_cast<uint32_t>(items + mine),
+                      static_cast<uint32_t>(segment), static_cast<uint32_t>(count[i]),
+                      static_cast<uint32_t>(mine / span * span), shift};
     if (i == 0)
       out->walk = CopyWalk{static_cast<uint32_t>(num_pairs), 0, k.chunks_per_tile, k.remap_end,
-                           k.run_shift, static_cast<uint32_t>(mine)};
+                           k.run_shift, k.end};
     else
       out->classes.at[i - 1] = k;
     items += mine;
