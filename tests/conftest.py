@@ -43,6 +43,17 @@ def aegkv_lib():
     return _lib.load()
 
 
+@pytest.fixture
+def always_staged(gpu):
+    """mode="staged" stages whatever runs a call leaves (by default a call of
+    short runs, as most tests' are, goes out as the DIRECT kernel)."""
+    from aegaeon_amd import _lib
+
+    prev = _lib.tune(_lib.TUNE_STAGED_SHORT_RUNS, 0)
+    yield
+    _lib.tune(_lib.TUNE_STAGED_SHORT_RUNS, prev)
+
+
 @pytest.fixture(scope="session")
 def gpu():
     import torch

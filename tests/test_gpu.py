@@ -16,7 +16,7 @@ import torch
 
 from aegaeon_amd import _lib, ops
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("always_staged")]
 
 
 MODES = ("direct", "staged")
@@ -261,8 +261,8 @@ def test_threads_swap_concurrently_on_their_own_streams(gpu):
 
 @pytest.mark.parametrize("mode", MODES)
 def test_unaligned_host_pool_vs_oracle(gpu, oracle, mode):
-    """A host pool starting 1 byte into its allocation forces the
-    byte-granular kernel path (and unaligned DMA in staged mode)."""
+    """A host pool starting 1 byte into its allocation forces the kernels for
+    any alignment (and unaligned DMA in staged mode)."""
     rng = np.random.default_rng(7)
     page = np.array([256, 512, 64], np.int64)
     cpu_off = np.array([0, 256, 768], np.int64)
@@ -369,7 +369,8 @@ def restore_tuning():
             _lib.TUNE_SWAP_OUT_WORKGROUPS, _lib.TUNE_SWAP_IN_WORKGROUPS, _lib.TUNE_NT_STORES,
             _lib.TUNE_STAGED_DMA_STREAMS, _lib.TUNE_STAGING_BYTES, _lib.TUNE_COPY_LDS_BYTES,
             _lib.TUNE_SWAP_UNROLL, _lib.TUNE_STAGED_WORKGROUPS, _lib.TUNE_STAGED_OVERLAP,
-            _lib.TUNE_SWAP_OUT_WORKGROUPS_UNCACHED, _lib.TUNE_COPY_LANES, _lib.TUNE_COPY_ORDER)
+            _lib.TUNE_SWAP_OUT_WORKGROUPS_UNCACHED, _lib.TUNE_COPY_LANES, _lib.TUNE_COPY_ORDER,
+            _lib.TUNE_STAGED_SHORT_RUNS)
     saved = {k: _lib.tune(k) for k in keys}
     yield
     for k, v in saved.items():
@@ -1002,8 +1003,10 @@ def _random_case(rng):
 def test_randomized_swaps_vs_oracle(gpu, oracle, restore_tuning, case):
     """Random layouts (groups, extents, TP ranks, byte and 16 B paths),
     both modes, random staging chunk sizes, DMA stream counts, overlap
-    settings and host-pool alignments: swap-out then swap-in to other ids,
-    each byte-equal to the oracle."""
+    settings and host-pool alignments, in one case of four with short STAGED
+    calls going DIRECT: swap-out then swap-in to other ids, each byte-equal to
+    the oracle."""
+    _lib.tune(_lib.TUNE_STAGED_SHORT_RUNS, int(np.random.default_rng(case).integers(0, 4) == 0))
     rng = np.random.default_rng(9000 + case)
     c = _random_case(rng)
     mode = MODES[case % 2]

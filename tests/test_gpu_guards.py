@@ -16,7 +16,7 @@ import torch
 
 from aegaeon_amd import ops
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("always_staged")]
 
 
 def _say(*a):

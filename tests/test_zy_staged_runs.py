@@ -22,13 +22,6 @@ def _say(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-@pytest.fixture()
-def always_staged():
-    prev = _lib.tune(_lib.TUNE_STAGED_SHORT_RUNS, 0)
-    yield
-    _lib.tune(_lib.TUNE_STAGED_SHORT_RUNS, prev)
-
-
 def test_the_rule_is_on_and_takes_0_or_1():
     assert _lib.tune(_lib.TUNE_STAGED_SHORT_RUNS) == 1
     with pytest.raises(ValueError):
