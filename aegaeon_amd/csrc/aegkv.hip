@@ -500,10 +500,12 @@ __global__ __launch_bounds__(256) void swap_inline_kernel(InlineSwap a) {
                                              (kernarg_i64*)(data + a.kpp_offset), a.walk);
 }
 
-// The classes of a walk where the launch put them. Indexed as a parameter they
-// would be copied to scratch memory. They come last of the arguments, so that
-// all a cache with one page size needs lies in one line of 64 bytes: behind
-// them, on a line border, copies of 0.6-4 ms took 1-3 us longer.
+// The classes of a walk behind the first, a kernel's last argument: none
+// (OneClass), or CopyClasses, read where the launch put them (indexed as a
+// parameter they would be copied to scratch memory). Kernels for caches with
+// one page size are built without them: looking for the class, and with 224
+// bytes more the arguments and the grid's size in several lines of 64 bytes,
+// took 0.1-0.5 % of a copy and 2-4 % of a probe.
 struct CopyArgs {
   const CopySeg* segs;
   const PairDesc* pairs;
@@ -513,9 +515,14 @@ struct CopyArgs {
 };
 static_assert(offsetof(CopyArgs, classes) == 64, "CopyArgs layout");
 typedef __attribute__((address_space(4))) const CopyClass kernarg_class;
-__device__ __forceinline__ kernarg_class* argument_classes() {
-  return (kernarg_class*)((kernarg_char*)__builtin_amdgcn_kernarg_segment_ptr() +
-                          offsetof(CopyArgs, classes));
+
+template <typename Classes>
+__device__ __forceinline__ auto argument_classes() {
+  if constexpr (sizeof(Classes) == sizeof(CopyClasses))
+    return (kernarg_class*)((kernarg_char*)__builtin_amdgcn_kernarg_segment_ptr() +
+                            offsetof(CopyArgs, classes));
+  else
+    return OneClass{};
 }
 
 // copy_blocks: one item is one chunk of one (segment, pair) tile. The host
@@ -547,14 +554,14 @@ __device__ __forceinline__ void copy_items(Segs segs, Pairs pairs, const CopyWal
   }
 }
 
-template <int WG, int U, bool VEC, bool NT_STORE>
+template <int WG, int U, bool VEC, bool NT_STORE, typename Classes>
 __global__ __launch_bounds__(WG) void copy_blocks_kernel(const CopySeg* __restrict__ segs,
                                                          const PairDesc* __restrict__ pairs,
                                                          CopyWalk walk,
                                                          const uint64_t* __restrict__ guard,
-                                                         CopyClasses) {
+                                                         Classes) {
   if (guard_set(guard)) return;
-  copy_items<WG, U, VEC, NT_STORE>(segs, pairs, walk, argument_classes());
+  copy_items<WG, U, VEC, NT_STORE>(segs, pairs, walk, argument_classes<Classes>());
 }
 
 // A short copy's whole descriptor (segment table, classes of the walk behind
@@ -578,14 +585,18 @@ static_assert(offsetof(InlineCopy, data) == 32 && sizeof(InlineCopy) <= 4096,
 typedef __attribute__((address_space(4))) const CopySeg kernarg_seg;
 typedef __attribute__((address_space(4))) const PairDesc kernarg_pair;
 
-template <int WG, bool VEC, bool NT_STORE>
+template <int WG, bool VEC, bool NT_STORE, typename Classes>
 __global__ __launch_bounds__(WG) void copy_blocks_inline_kernel(InlineCopy a) {
   // the tables are indexed where the launch put them: `a` is the kernel's
   // only argument and starts its argument segment
   kernarg_char* data =
       (kernarg_char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(InlineCopy, data);
-  copy_items<WG, 1, VEC, NT_STORE>((kernarg_seg*)data, (kernarg_pair*)(data + a.pair_offset),
-                                   a.walk, (kernarg_class*)(data + a.class_offset));
+  kernarg_seg* segs = (kernarg_seg*)data;
+  kernarg_pair* pairs = (kernarg_pair*)(data + a.pair_offset);
+  if constexpr (sizeof(Classes) == sizeof(CopyClasses))
+    copy_items<WG, 1, VEC, NT_STORE>(segs, pairs, a.walk, (kernarg_class*)(data + a.class_offset));
+  else
+    copy_items<WG, 1, VEC, NT_STORE>(segs, pairs, a.walk, OneClass{});
 }
 
 // Measurement twins of copy_blocks_kernel (aegkv_copy_probe): the same
@@ -598,17 +609,17 @@ __global__ __launch_bounds__(WG) void copy_blocks_inline_kernel(InlineCopy a) {
 constexpr int PROBE_READ = 1;
 constexpr int PROBE_WRITE = 2;
 
-template <int WG, int U, int KIND, bool NT_STORE>
+template <int WG, int U, int KIND, bool NT_STORE, typename Classes>
 __global__ __launch_bounds__(WG) void copy_probe_kernel(const CopySeg* __restrict__ segs,
                                                         const PairDesc* __restrict__ pairs,
                                                         CopyWalk walk, uint32_t* sink,
-                                                        uint32_t magic, CopyClasses) {
+                                                        uint32_t magic, Classes) {
   constexpr int64_t kChunk = Shape<WG, U>::kChunk;
   const uint32_t tid = threadIdx.x;
   v4u acc = {0u, 0u, 0u, 0u};
   const v4u pattern = {tid, blockIdx.x, 0x5a5a5a5au, magic};
   for (uint32_t w = blockIdx.x; w < walk.num_items; w += gridDim.x) {
-    const CopyItem it = copy_item(walk, argument_classes(), w);
+    const CopyItem it = copy_item(walk, argument_classes<Classes>(), w);
     const PairDesc pr = pairs[it.pair];
     const CopySeg seg = segs[it.segment];
     const int64_t begin = static_cast<int64_t>(it.chunk) * kChunk;
@@ -1242,8 +1253,13 @@ template <int WG, int U, bool VEC, bool NT>
 hipError_t launch_copy_t(int64_t grid, unsigned lds, hipStream_t st, const CopySeg* s,
                          const PairDesc* p, const CopyLayout& l, const uint64_t* guard) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
-  hipLaunchKernelGGL((copy_blocks_kernel<WG, U, VEC, NT>), dim3(static_cast<uint32_t>(grid)),
-                     dim3(WG), lds, st, s, p, l.walk, guard, l.classes);
+  const dim3 g(static_cast<uint32_t>(grid));
+  if (l.num_classes)
+    hipLaunchKernelGGL((copy_blocks_kernel<WG, U, VEC, NT, CopyClasses>), g, dim3(WG), lds, st, s,
+                       p, l.walk, guard, l.classes);
+  else
+    hipLaunchKernelGGL((copy_blocks_kernel<WG, U, VEC, NT, OneClass>), g, dim3(WG), lds, st, s, p,
+                       l.walk, guard, OneClass{});
   return hipGetLastError();
 }
 
@@ -1269,23 +1285,27 @@ hipError_t launch_copy(ShapeSel sh, bool vec, bool nt, int64_t grid, unsigned ld
 }
 
 template <int WG, bool VEC, bool NT>
-hipError_t launch_inline_t(int64_t grid, hipStream_t st, const InlineCopy& a) {
+hipError_t launch_inline_t(bool one_class, int64_t grid, hipStream_t st, const InlineCopy& a) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
-  hipLaunchKernelGGL((copy_blocks_inline_kernel<WG, VEC, NT>),
-                     dim3(static_cast<uint32_t>(grid)), dim3(WG), 0, st, a);
+  const dim3 g(static_cast<uint32_t>(grid));
+  if (one_class)
+    hipLaunchKernelGGL((copy_blocks_inline_kernel<WG, VEC, NT, OneClass>), g, dim3(WG), 0, st, a);
+  else
+    hipLaunchKernelGGL((copy_blocks_inline_kernel<WG, VEC, NT, CopyClasses>), g, dim3(WG), 0, st,
+                       a);
   return hipGetLastError();
 }
 
-hipError_t launch_inline(int lanes, bool vec, bool nt, int64_t grid, hipStream_t st,
-                         const InlineCopy& a) {
+hipError_t launch_inline(int lanes, bool vec, bool nt, bool one, int64_t grid,
+                         hipStream_t st, const InlineCopy& a) {
   if (!vec)
-    return nt ? launch_inline_t<64, false, true>(grid, st, a)
-              : launch_inline_t<64, false, false>(grid, st, a);
+    return nt ? launch_inline_t<64, false, true>(one, grid, st, a)
+              : launch_inline_t<64, false, false>(one, grid, st, a);
   if (lanes == 64)
-    return nt ? launch_inline_t<64, true, true>(grid, st, a)
-              : launch_inline_t<64, true, false>(grid, st, a);
-  return nt ? launch_inline_t<256, true, true>(grid, st, a)
-            : launch_inline_t<256, true, false>(grid, st, a);
+    return nt ? launch_inline_t<64, true, true>(one, grid, st, a)
+              : launch_inline_t<64, true, false>(one, grid, st, a);
+  return nt ? launch_inline_t<256, true, true>(one, grid, st, a)
+            : launch_inline_t<256, true, false>(one, grid, st, a);
 }
 
 template <int WG, int U, int KIND, bool NT>
@@ -1293,8 +1313,13 @@ hipError_t launch_probe_t(int64_t grid, unsigned lds, hipStream_t st, const Copy
                           const PairDesc* p, const CopyLayout& l, uint32_t* sink,
                           uint32_t magic) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
-  hipLaunchKernelGGL((copy_probe_kernel<WG, U, KIND, NT>), dim3(static_cast<uint32_t>(grid)),
-                     dim3(WG), lds, st, s, p, l.walk, sink, magic, l.classes);
+  const dim3 g(static_cast<uint32_t>(grid));
+  if (l.num_classes)
+    hipLaunchKernelGGL((copy_probe_kernel<WG, U, KIND, NT, CopyClasses>), g, dim3(WG), lds, st, s,
+                       p, l.walk, sink, magic, l.classes);
+  else
+    hipLaunchKernelGGL((copy_probe_kernel<WG, U, KIND, NT, OneClass>), g, dim3(WG), lds, st, s, p,
+                       l.walk, sink, magic, OneClass{});
   return hipGetLastError();
 }
 
@@ -2120,7 +2145,8 @@ int copy_inline(const CopyPlan& p, const Tunables& t, int num_cus, int32_t num_s
                  dst_bases, page_bytes, num_pairs, src_ids, dst_ids, t.copy_order, tmp);
   std::memcpy(a.data + class_offset, p.lay.classes.at, sizeof(CopyClass) * p.lay.num_classes);
   const int64_t grid = launch_grid(t.copy_wgs_per_cu * num_cus, p.lay.walk.num_items, p.sh.wg);
-  const hipError_t e = launch_inline(p.sh.wg, p.vec, t.nt_stores != 0, grid, stream, a);
+  const hipError_t e = launch_inline(p.sh.wg, p.vec, t.nt_stores != 0,
+                                     p.lay.num_classes == 0, grid, stream, a);
   if (e != hipSuccess) return hip_fail(e, "copy_blocks_inline_kernel launch");
   *launched = true;
   return 0;

@@ -78,8 +78,7 @@ inline int64_t tile_chunks(int64_t page, int64_t chunk, bool vec) {
 // others' workgroups were empty: beside 63 tensors of 16 KiB pages one of 160
 // KiB left 88 % of them so, and 1500 pairs took 2.29 ms where they now take
 // 0.58 (6.2 TB/s, read plus written); 160 KiB, 16 KiB and 512 bytes in equal
-// number 2.66 -> 1.69 ms, 41,984 and 8,448 bytes 0.96 -> 0.79. A cache with
-// one page size pays one scalar comparison an item.
+// number 2.66 -> 1.69 ms, 41,984 and 8,448 bytes 0.96 -> 0.79.
 struct alignas(32) CopyClass {
   uint32_t first_item, end;
   uint32_t first_segment, chunks_per_tile;
@@ -101,6 +100,8 @@ struct CopyClasses {  // the others
   CopyClass at[kCopyClasses - 1];
 };
 
+struct OneClass {};  // in their place where there are none
+
 struct CopyItem {
   uint32_t pair, segment, chunk, last;
 };
@@ -118,10 +119,13 @@ AEGKV_HOST_DEVICE CopyItem class_item(uint32_t num_pairs, uint32_t first_segment
 }
 
 // Item w (below num_items). `classes`: those behind the first one.
+AEGKV_HOST_DEVICE CopyItem copy_item(const CopyWalk& k, OneClass, uint32_t w) {
+  return class_item(k.num_pairs, 0, k.chunks_per_tile, k.remap_end, k.run_shift, w);
+}
+
 template <typename Classes>
 AEGKV_HOST_DEVICE CopyItem copy_item(const CopyWalk& k, Classes classes, uint32_t w) {
-  if (w < k.first_end)
-    return class_item(k.num_pairs, 0, k.chunks_per_tile, k.remap_end, k.run_shift, w);
+  if (w < k.first_end) return copy_item(k, OneClass{}, w);
   uint32_t i = 0;
   while (w >= classes[i].end) ++i;
   return class_item(k.num_pairs, classes[i].first_segment, classes[i].chunks_per_tile,

@@ -37,7 +37,8 @@ double walk(const std::vector<int64_t>& pages, int64_t pairs, bool vec, int shif
   std::vector<std::vector<std::pair<int64_t, int64_t>>> got(static_cast<size_t>(S * pairs));
   int64_t empty = 0;
   for (uint32_t w = 0; w < l.walk.num_items; ++w) {
-    const CopyItem it = copy_item(l.walk, l.classes.at, w);
+    const CopyItem it = l.num_classes ? copy_item(l.walk, l.classes.at, w)
+                                      : copy_item(l.walk, OneClass{}, w);
     CHECK(it.segment < static_cast<uint32_t>(S) && it.pair < pairs && it.chunk <= it.last);
     const int64_t page = held[it.segment];
     int64_t begin = static_cast<int64_t>(it.chunk) * kChunk;
