@@ -5,14 +5,14 @@
 //   * swap-in   : composite host pages -> device K/V tiles
 //   * copy_blocks: device block -> device block, every backing tensor
 //
-// One persistent "tile mover" kernel family does all of it. A work item is
-// one 16 B-per-lane chunk of one (entry, segment) tile; a workgroup of 256
-// lanes moves CHUNK = 256 * 16 * UNROLL bytes per item with all UNROLL loads
-// issued before the first store. Items are entry-major so consecutive items
-// walk one composite host page in address order (good for PCIe write
-// combining and host DRAM pages); link-bound swaps run a few persistent
-// workgroups that stride over the item space, HBM-bound moves one workgroup
-// per item.
+// One "tile mover" kernel family does all of it. A work item is one chunk of
+// one tile (a segment's bytes of one entry or pair): WG lanes move WG * 16 * U
+// bytes with all U loads issued before the first store. Swaps are link-bound:
+// a few persistent workgroups of 256 lanes stride over items in entry order,
+// so that consecutive ones walk one composite host page in address order (good
+// for PCIe write combining and host DRAM pages). Copies are HBM-bound: one
+// workgroup of 64 or 256 lanes (1024 for whole tiles on masked streams) per
+// item, segment by segment (copy_walk.h).
 //
 // Two host-transfer designs share the kernel:
 //   DIRECT: the "host side" pointer is the pinned host pool itself (mapped
@@ -776,8 +776,9 @@ ShapeSel auto_shape(int64_t page) {
 // lanes idle in the last one. In the order of copy_item, few bytes per item
 // keep what the chip writes at any moment close together: 160 KiB tiles run
 // at 6.45 TB/s (streaming stores) with 4 KiB items, 6.18 with 8 or 16 KiB,
-// 6.03 with one item a tile; 12.5 KiB tiles at 5.69 with 4 KiB items and 6.02 with 1 KiB, 1 KiB
-// tiles at 3.84 and 6.19. On multiples of 4 KiB the two are within 1 %.
+// 6.03 with one item a tile; 12.5 KiB tiles at 5.69 with 4 KiB items and 6.02
+// with 1 KiB, 1 KiB tiles at 3.84 and 6.19. On multiples of 4 KiB the two are
+// within 1 %.
 //
 // One load per lane keeps 32 KiB in flight on a CU, which fills the chip's
 // memory system only with all CUs. A stream masked to some of them
@@ -2218,11 +2219,11 @@ int copy_core(int32_t num_segments, void* const* src_bases, void* const* dst_bas
 // a fixed device array every GPU holds for the life of the process, instead
 // of the library's upload ring; it travels in the kernel arguments of small
 // fill launches, or of the copy itself where it is short (copy_inline), so a
-// graph that captures the call replays its own descriptor. The ids are checked with fixed host arrays instead of a
-// block-indexed map. Nothing is allocated on the host or the device. Every
-// call on a device shares that device's array, so calls that overlap on one
-// device (different streams, or threads, or a graph replayed beside other
-// calls) race; calls on one stream are ordered.
+// graph that captures the call replays its own descriptor. The ids are checked
+// with fixed host arrays instead of a block-indexed map. Nothing is allocated
+// on the host or the device. Every call on a device shares that device's array,
+// so calls that overlap on one device (different streams, or threads, or a
+// graph replayed beside other calls) race; calls on one stream are ordered.
 
 constexpr int32_t kNoAllocMaxSegments = 1024;
 constexpr int64_t kNoAllocMaxPairs = 65536;
@@ -2297,7 +2298,8 @@ hipError_t noalloc_fill(char* dst, const unsigned char* src, int32_t num_segment
     a.num_pairs = static_cast<uint32_t>(
         std::min<int64_t>(num_pairs - p, static_cast<int64_t>((kFillBytes - used) / pair_bytes)));
     FillSeg* fs = reinterpret_cast<FillSeg*>(a.data);
-    for (uint32_t i = 0; i < a.num_segs; ++i) fs[i] = FillSeg{segs[s + i].dst, segs[s + i].page_bytes};
+    for (uint32_t i = 0; i < a.num_segs; ++i)
+      fs[i] = FillSeg{segs[s + i].dst, segs[s + i].page_bytes};
     if (a.wide) {
       std::memcpy(a.data + used, pairs + p, a.num_pairs * pair_bytes);
     } else {

@@ -1505,7 +1505,7 @@ def main():
         "copy_blocks_cu_partition": None if part is None else dict(part, what=(
             "the same copy on a dedicated stream masked to CUs 0-23 of every XCD "
             "(DedicatedStream(cu_mask=xcd_cu_mask(24))), a caller's choice, not the roofline "
-            "value: one tile in flight per CU on 192 CUs instead of 256")),
+            "value: whole tiles, one in flight per CU, on 192 CUs")),
         "link_roofline": {
             "bound": "host-link (measured)",
             "kernel": "swap_tiles_kernel",

@@ -242,10 +242,10 @@ int aegkv_copy_blocks(int32_t num_segments, void* const* segment_bases,
  * 1,081,344 bytes that each GPU the library runs on holds until the process
  * ends, written there by small fill kernels whose arguments carry the
  * descriptor (3776 bytes per launch, 8 a pair; 4096 pairs over 80 segments
- * take 10 launches), or, for a short call (94 pairs over 72 segments), in
- * the arguments of the copy itself. A graph that captures the call therefore replays the
- * descriptor it captured, whatever calls ran since. The launches cost host
- * time: measured 0.33 ms per call for 4096 pairs over 80 segments and
+ * take 10 launches), or, for a short call (up to 94 pairs over 72 segments of
+ * one page size), in the arguments of the copy itself. A graph that captures
+ * the call therefore replays the descriptor it captured, whatever calls ran
+ * since. The launches cost host time: measured 0.33 ms per call for 4096 pairs over 80 segments and
  * 6.1 ms for 65536 pairs, against 0.05 and 0.41 ms for aegkv_copy_blocks; the
  * same for up to a few hundred pairs. Limits: at most 1024
  * segments and 65536 pairs per call (AEGKV_ENOMEM beyond, nothing
