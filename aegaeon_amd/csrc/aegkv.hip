@@ -575,13 +575,13 @@ __global__ __launch_bounds__(WG) void copy_blocks_kernel(const CopySeg* __restri
 // kInlineBytes keeps all arguments, hidden ones among them, within 4 KiB: 72
 // segments and 94 pairs.
 constexpr uint32_t kInlineBytes = 3808;
-struct alignas(16) InlineCopy {
+struct alignas(32) InlineCopy {
   CopyWalk walk;
   uint32_t class_offset, pair_offset;  // from data
   unsigned char data[kInlineBytes];
 };
-static_assert(offsetof(InlineCopy, data) == 32 && sizeof(InlineCopy) <= 4096,
-              "InlineCopy layout");
+static_assert(offsetof(InlineCopy, data) % alignof(CopyClass) == 0 && sizeof(InlineCopy) <= 3840,
+              "InlineCopy layout: 4 KiB of arguments, 256 bytes of them hidden ones");
 typedef __attribute__((address_space(4))) const CopySeg kernarg_seg;
 typedef __attribute__((address_space(4))) const PairDesc kernarg_pair;
 
