@@ -280,8 +280,8 @@ using ShapeWords = Words<!NT_STORE ? kPlain : U == 1 && WG <= 256 ? kThrough : k
 // (252 VGPRs for U = 8, and with 1024 lanes scratch memory: 128 KiB tiles
 // copied at 1.3 TB/s). A lane's store stands under its load's own condition:
 // under two equal ones the compiler takes a load for possibly unfinished
-// behind them, and a loop over items then waits for all of an item's stores
-// before it starts the next (stores_first is where that is wanted).
+// behind them, and a loop over items then waits for an item's stores wherever
+// it next uses the register (wait_for_stores is where that is wanted).
 template <int WG, int U, typename Out>
 __device__ __forceinline__ void move_tail16(const gv4u* s, const Out& d, uint32_t i,
                                             uint32_t n16) {
@@ -389,26 +389,20 @@ __device__ __forceinline__ bool guard_set_at_source(const uint64_t* guard) {
   return set != 0;
 }
 
-// Wait for this wave's stores (and loads) to complete.
+// The persistent workgroups of a swap or a weight load wait for an item's
+// stores before they load the next item. Without that the same grid keeps
+// twice the requests to the host in the memory queues, and what else uses HBM
+// or the link beside it waits behind them: a copy beside a swap-out of 24 / 32
+// workgroups runs at 6.0 / 5.8 TB/s, 4.5 / 2.1 without; beside a swap-in of 48
+// at 5.9, 2.2 without; beside both at 24 / 24 at 5.9, 3.6 without. Both
+// directions at 16 / 16 reach 94.3 GB/s (88-92), a switch at the default grids
+// 11.6 ms (11.7), with a weight load beside it 22.4 (23.2).
+// It costs swaps both ways at 20 to 48 workgroups of two loads, or 12 to 16 of
+// four, with nothing beside them (24 / 24 on streams over all CUs 14.9 ms a
+// switch, 12.9 without; 32 / 32 13.6, 12.4), and one direction over 4 to 8
+// workgroups (4: 32 GB/s, 40 without).
 __device__ __forceinline__ void wait_for_stores() {
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), the other counters as they are
-}
-
-// Whether the persistent workgroups of a swap or a weight load wait for an
-// item's stores before they load the next. With a lot in flight that shares
-// the link better between both directions and a weight load; with less it
-// leaves the link idle. A model switch of 2 x 550 MB each way at equal grids
-// both ways, waiting -> not (ms): 24 workgroups of two loads (192 KiB in
-// flight) 14.8 -> 12.9, 20 of two 14.8 -> 12.8, 32 of two 13.3 -> 12.4, 16 of
-// four 14.0 -> 12.7, 48 of two (384 KiB) 12.4 -> 12.1; 64 of four (1 MiB)
-// 11.8 -> 12.0, the default grids 11.6 -> 11.7, with a weight load beside them
-// 22.4 -> 23.2. One direction alone at 4 of two 14.7 -> 11.9, from 16 up within
-// 2 %. (Below: 16 of two both ways 11.4 -> 11.9, 8 of four 11.9 -> 12.7, which
-// is one point of a steep curve and not followed.)
-constexpr int64_t kStoresFirstBytes = int64_t(512) << 10;
-
-bool stores_first(int64_t grid, int64_t items, int64_t chunk) {
-  return grid < items && grid * chunk >= kStoresFirstBytes;
 }
 
 // What a swap kernel needs beside its tables.
@@ -416,7 +410,6 @@ struct SwapWalk {
   char* host_base;
   int64_t host_stride, host_rank_offset;
   uint32_t num_segs, num_items, chunks_per_tile;
-  uint32_t stores_first;
 };
 
 // Swap tile mover. Item w -> (entry e, segment s, chunk c), entry-major.
@@ -443,9 +436,9 @@ __device__ __forceinline__ void swap_items(Segs segs, Ents ents, Kpp kpp, const 
                  segs[s].host_offset + off;
     const char* src = TO_HOST ? dev : host;
     char* dst = TO_HOST ? host : dev;
-    if (k.stores_first) wait_for_stores();
     if (VEC) {
       const int64_t begin = static_cast<int64_t>(c) * kChunk;
+      wait_for_stores();
       if (begin >= len) continue;
       const uint32_t nbytes =
           static_cast<uint32_t>((len - begin < kChunk) ? (len - begin) : kChunk);
@@ -669,8 +662,7 @@ static_assert(sizeof(SliceDesc) == 32, "SliceDesc layout");
 // slices are dropped on the host, so every slice has at least one item.
 template <int WG, int U, bool VEC, bool NT_STORE>
 __global__ __launch_bounds__(WG) void slices_kernel(const SliceDesc* __restrict__ slices,
-                                                    uint32_t num_slices, uint32_t num_items,
-                                                    uint32_t stores_first) {
+                                                    uint32_t num_slices, uint32_t num_items) {
   constexpr int64_t kChunk = Shape<WG, U>::kChunk;
   for (uint32_t w = blockIdx.x; w < num_items; w += gridDim.x) {
     uint32_t lo = 0, hi = num_slices - 1;
@@ -683,11 +675,11 @@ __global__ __launch_bounds__(WG) void slices_kernel(const SliceDesc* __restrict_
     }
     const SliceDesc sl = slices[lo];
     const uint32_t c = static_cast<uint32_t>(static_cast<int64_t>(w) - sl.first_item);
-    if (stores_first) wait_for_stores();
     if (VEC) {
       const int64_t begin = static_cast<int64_t>(c) * kChunk;
       const uint32_t nbytes =
           static_cast<uint32_t>((sl.bytes - begin < kChunk) ? (sl.bytes - begin) : kChunk);
+      wait_for_stores();
       move_chunk16<WG, U, NT_STORE>(sl.src + begin, sl.dst + begin, nbytes);
     } else {
       const uint32_t last = static_cast<uint32_t>((sl.bytes - 1) / kChunk);
@@ -1347,19 +1339,18 @@ hipError_t launch_slices(bool vec, bool nt, int64_t grid, hipStream_t st,
                          const SliceDesc* slices, uint32_t num_slices, uint32_t items) {
   (void)hipGetLastError();  // clear a stale error: the check below is for this launch
   const dim3 g(static_cast<uint32_t>(grid));
-  const uint32_t first = stores_first(grid, items, int64_t(256) * 16 * 2);
   if (!vec && nt)
     hipLaunchKernelGGL((slices_kernel<256, 2, false, true>), g, dim3(256), 0, st, slices,
-                       num_slices, items, first);
+                       num_slices, items);
   else if (!vec)
     hipLaunchKernelGGL((slices_kernel<256, 2, false, false>), g, dim3(256), 0, st, slices,
-                       num_slices, items, first);
+                       num_slices, items);
   else if (nt)
     hipLaunchKernelGGL((slices_kernel<256, 2, true, true>), g, dim3(256), 0, st, slices,
-                       num_slices, items, first);
+                       num_slices, items);
   else
     hipLaunchKernelGGL((slices_kernel<256, 2, true, false>), g, dim3(256), 0, st, slices,
-                       num_slices, items, first);
+                       num_slices, items);
   return hipGetLastError();
 }
 
@@ -1542,8 +1533,7 @@ int enqueue_swap_kernel(DeviceCtx* ctx, const SwapLayout& L, const SwapList& E,
   if (items < 0) return too_many_items(n, S, cpt, "entries");
   const int64_t grid = launch_grid(wgs, items, sh.wg);
   const SwapWalk walk{host_side, host_stride, host_rank_off, static_cast<uint32_t>(S),
-                      static_cast<uint32_t>(items), static_cast<uint32_t>(cpt),
-                      stores_first(grid, items, sh.chunk())};
+                      static_cast<uint32_t>(items), static_cast<uint32_t>(cpt)};
   // Non-temporal stores only where the destination is HBM: plain stores to
   // the host pool measured faster (no L2 residency to avoid there).
   const bool nt = t.nt_stores != 0 && !(!is_swap_in && !staged);

@@ -685,10 +685,9 @@ def test_copy_walk_covers_every_item_once(gpu, page, segs, pairs):
 
 @pytest.mark.parametrize("workgroups,unroll", [(1, 2), (31, 4), (32, 4), (63, 2), (64, 2), (65, 2),
                                                (128, 1), (127, 1)])
-def test_persistent_grids_around_the_wait_for_stores(gpu, restore_tuning, workgroups, unroll):
-    """From 512 KiB in flight the workgroups of swaps and weight loads wait
-    for an item's stores before they load the next; the bytes are the same on
-    both sides of that line, in whole items and tails, aligned or not."""
+def test_persistent_grids_of_swaps_and_weight_loads(gpu, restore_tuning, workgroups, unroll):
+    """Workgroups that take one item after another move the same bytes at any
+    grid, in whole items and tails, aligned or not."""
     _say("persistent grids", workgroups, unroll)
     for key in (_lib.TUNE_SWAP_OUT_WORKGROUPS, _lib.TUNE_SWAP_IN_WORKGROUPS):
         _lib.tune(key, workgroups)
