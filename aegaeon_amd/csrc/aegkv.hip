@@ -278,17 +278,31 @@ using ShapeWords = Words<!NT_STORE ? kPlain : U == 1 && WG <= 256 ? kThrough : k
 // Recursion keeps every value in registers of its own: an array of U values
 // filled under conditions became one wide value that was copied whole at each
 // (252 VGPRs for U = 8, and with 1024 lanes scratch memory: 128 KiB tiles
-// copied at 1.3 TB/s). A lane's store stands under its load's own condition:
-// under two equal ones the compiler takes a load for possibly unfinished
-// behind them, and a loop over items then waits for an item's stores wherever
-// it next uses the register (wait_for_stores is where that is wanted).
+// copied at 1.3 TB/s).
+//
+// Load and store stand under conditions of their own, so the compiler takes a
+// tail's load for possibly unfinished behind them, and the loops over items of
+// swaps and weight loads wait for all of an item's memory operations, its
+// stores among them, where they next use the register: before the next item's
+// loads. That wait is wanted. Without it (the store nested under
+// its load's condition) the same grid keeps twice the requests to the host in
+// the memory queues, and what else uses HBM or the link waits behind them: a
+// copy beside a swap-out of 24 / 32 workgroups runs at 6.0 / 5.8 TB/s, 4.5 / 2.1
+// without; beside a swap-in of 48 at 5.9, 2.2 without; beside both at 24 / 24 at
+// 5.9, 3.6 without. Both directions at 16 / 16 reach 92-95 GB/s (88-92), a switch
+// at the default grids 11.6 ms (11.7), with a weight load beside it 22.4 (23.2).
+// It costs swaps both ways at 20 to 48 workgroups of two loads, or 12 to 16 of
+// four, with nothing beside them (24 / 24 14.9 ms a switch, 12.9 without; 32 / 32
+// 13.6, 12.4), and one direction over 4 to 8 workgroups (4: 32 GB/s, 40 without).
+// Asked for in the source right before the loads, behind the addresses, it made
+// both ways at 12 to 32 workgroups another 4-9 % slower.
 template <int WG, int U, typename Out>
 __device__ __forceinline__ void move_tail16(const gv4u* s, const Out& d, uint32_t i,
                                             uint32_t n16) {
-  if (i >= n16) return;  // nor has the lane any later word
-  const v4u x = __builtin_nontemporal_load(s + i);
+  v4u x;
+  if (i < n16) x = __builtin_nontemporal_load(s + i);
   if constexpr (U > 1) move_tail16<WG, U - 1>(s, d, i + WG, n16);
-  d.put(i, x);
+  if (i < n16) d.put(i, x);
 }
 
 // Move nbytes (multiple of 16, at most one chunk) with 16 B per lane. A full
@@ -389,22 +403,6 @@ __device__ __forceinline__ bool guard_set_at_source(const uint64_t* guard) {
   return set != 0;
 }
 
-// The persistent workgroups of a swap or a weight load wait for an item's
-// stores before they load the next item. Without that the same grid keeps
-// twice the requests to the host in the memory queues, and what else uses HBM
-// or the link beside it waits behind them: a copy beside a swap-out of 24 / 32
-// workgroups runs at 6.0 / 5.8 TB/s, 4.5 / 2.1 without; beside a swap-in of 48
-// at 5.9, 2.2 without; beside both at 24 / 24 at 5.9, 3.6 without. Both
-// directions at 16 / 16 reach 94.3 GB/s (88-92), a switch at the default grids
-// 11.6 ms (11.7), with a weight load beside it 22.4 (23.2).
-// It costs swaps both ways at 20 to 48 workgroups of two loads, or 12 to 16 of
-// four, with nothing beside them (24 / 24 on streams over all CUs 14.9 ms a
-// switch, 12.9 without; 32 / 32 13.6, 12.4), and one direction over 4 to 8
-// workgroups (4: 32 GB/s, 40 without).
-__device__ __forceinline__ void wait_for_stores() {
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), the other counters as they are
-}
-
 // What a swap kernel needs beside its tables.
 struct SwapWalk {
   char* host_base;
@@ -438,7 +436,6 @@ __device__ __forceinline__ void swap_items(Segs segs, Ents ents, Kpp kpp, const 
     char* dst = TO_HOST ? host : dev;
     if (VEC) {
       const int64_t begin = static_cast<int64_t>(c) * kChunk;
-      wait_for_stores();
       if (begin >= len) continue;
       const uint32_t nbytes =
           static_cast<uint32_t>((len - begin < kChunk) ? (len - begin) : kChunk);
@@ -679,7 +676,6 @@ __global__ __launch_bounds__(WG) void slices_kernel(const SliceDesc* __restrict_
       const int64_t begin = static_cast<int64_t>(c) * kChunk;
       const uint32_t nbytes =
           static_cast<uint32_t>((sl.bytes - begin < kChunk) ? (sl.bytes - begin) : kChunk);
-      wait_for_stores();
       move_chunk16<WG, U, NT_STORE>(sl.src + begin, sl.dst + begin, nbytes);
     } else {
       const uint32_t last = static_cast<uint32_t>((sl.bytes - 1) / kChunk);
